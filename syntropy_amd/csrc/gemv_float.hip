@@ -1,0 +1,261 @@
+// Gemv over F16 and BF16 weights on gfx950 (crates/kernels-cpu/src/gemv/portable.rs:30-45
+// float_rows with the fold of gemv.rs:506-516): per output, 32 F32 accumulators; element i goes
+// into accumulator i % 32 with one fused multiply-add, in increasing i; then the halving fold
+// acc[j] += acc[j + h] for h = 16, 8, 4, 2, 1.  The activations stay F32 (no quantization).
+//
+// The accumulators on the matrix cores.  v_mfma_f32_4x4x1_16b_f32 is sixteen independent 4 x 4
+// outer products with one product a sum, each D = fma(A, B, C): one fused multiply-add, rounded
+// once, subnormals and zero signs kept (checked against fmaf on the device over random finite
+// operands, subnormal results among them).  So the sixteen blocks are sixteen accumulators of
+// 4 weight rows x 4 activation rows: lane l = 4 b + i holds, of weight row i of the tile, the
+// dword of elements 32 m + 2 b and + 1 (accumulators 2 b and 2 b + 1: two instructions), and of
+// activation row i the same two F32 values.
+//
+// What bounds it.  The weights' bytes, read once for up to 16 activation rows.  A wavefront takes
+// R tiles of 4 weight rows x C tiles of 4 activation rows over the whole row length, KC elements a
+// stage.  Weights (each wavefront its own rows) and activation rows (one set for the workgroup) are
+// copied into LDS by global_load_lds in whole kilobytes of a row, NS - 1 stages ahead.
+// Measured on 32064 x 4096 F16 (263 MB), against one 16-byte load a lane and F32 FMAs on four
+// activation rows a pass: 54 us (4.9 TB/s) against 78 at one row, 75 against 288 at 9, 87 against
+// 450 at 16, 174 against 833 at 32.  4096 x 4096: 9.6 against 41 us at one row.
+#include <type_traits>
+
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace syn {
+
+typedef float v4f_f __attribute__((ext_vector_type(4)));
+
+template <int C, int R, int WV, int KC, int NS>
+struct GfCfg {
+    static constexpr int MC = KC / 32;             // steps of 32 elements a stage
+    static constexpr int RPC = 1024 / (2 * KC);    // weight rows a copy instruction moves (1 KB)
+    // A piece of LDS a copy instruction fills, and 32 bytes more: the four weight rows of a tile (one
+    // dword a lane) and the four activation rows of a tile (two dwords) then start 32 bytes apart
+    // modulo the 128 bytes that a group of lanes reads at once, which no two lanes share a bank in.
+    static constexpr int WPIECE = 1024 + 32;
+    static constexpr int WCOPIES = 4 * R / RPC;    // per wavefront a stage
+    static constexpr int WBYTES = WCOPIES * WPIECE;
+    static constexpr int XROW = 4 * KC + 32;
+    static constexpr int XPIECES = 4 * C * KC * 4 / 1024;
+    static constexpr int XCOPIES = (XPIECES + WV - 1) / WV;
+    static constexpr int STAGE = WV * WBYTES + 4 * C * XROW;
+    static constexpr int COPIES = WCOPIES + XCOPIES;
+    static constexpr size_t LDS = (size_t)NS * STAGE;
+    static_assert(RPC >= 1 && R % RPC == 0, "a copy takes row i of RPC tiles");
+    static_assert(COPIES * (NS - 2) <= 63, "the wait count fits vmcnt");
+    static_assert(LDS <= 160 * 1024, "LDS");
+};
+
+// VEC: rows of whole 16-byte pieces at 16-byte aligned addresses, copied by global_load_lds; else
+// element by element through registers.
+template <int BF16, int VEC, int C, int R, int WV, int KC, int NS>
+__global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __restrict__ W, int n_out, int k,
+                                                          const float* __restrict__ x, int rows,
+                                                          float* __restrict__ y,
+                                                          const uint32_t* __restrict__ active, int groups) {
+    using G = GfCfg<C, R, WV, KC, NS>;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    rows = active_rows(active, 0, rows);
+    // activation groups of the same weight rows run on the same XCD (workgroups go to the 8 XCDs
+    // in turn), one after the other, so that the later ones find the weights in its L2
+    const int wb = groups == 1 ? (int)blockIdx.x : 8 * ((int)blockIdx.x / (8 * groups)) + (int)(blockIdx.x & 7);
+    const int t0 = groups == 1 ? 0 : 4 * C * (((int)blockIdx.x >> 3) % groups);
+    if (t0 >= rows) return;  // uniform
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b = lane >> 2, i = lane & 3;
+    const int row0 = (wb * WV + wave) * 4 * R;
+    const int ns = (k + KC - 1) / KC;
+    const uint32_t rb = 2u * (uint32_t)k;
+    v4f_f acc[R][C][2];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[r][c][j] = v4f_f{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // weight copy u: row i' = u % 4 of tiles RPC (u / 4) .. + RPC - 1, 64 / RPC lanes each; rows past
+    // the matrix re-read its last one, bytes past a row its last piece (neither is used)
+    const uint8_t* wbase = W + (uint64_t)(row0 < n_out ? row0 : n_out - 1) * rb;
+    const int last = n_out - 1 - (row0 < n_out ? row0 : n_out - 1);  // the last row, from wbase
+    auto issue = [&](int s) {
+        uint8_t* st = lds + (s % NS) * G::STAGE;
+        const int sc = s < ns ? s : ns - 1;  // a stage past the row repeats the last, so that the counts stay
+#pragma unroll
+        for (int u = 0; u < G::WCOPIES; ++u) {
+            const int tr = G::RPC * (u / 4) + lane / (64 / G::RPC);
+            const int row = 4 * tr + (u & 3) < last ? 4 * tr + (u & 3) : last;
+            if constexpr (VEC) {
+                const uint32_t at = 2u * KC * (uint32_t)sc + 16u * (uint32_t)(lane % (64 / G::RPC));
+                lds_dma16((uint32_t)row * rb + (at < rb ? at : rb - 16), wbase,
+                          lds_addr(st) + (uint32_t)(wave * G::WBYTES + u * G::WPIECE));
+            } else {
+                const int e = KC * sc + 8 * (lane % (64 / G::RPC));
+                const uint16_t* src = reinterpret_cast<const uint16_t*>(wbase) + (int64_t)row * k;
+                uint16_t* dst = reinterpret_cast<uint16_t*>(st + wave * G::WBYTES + u * G::WPIECE) + 8 * lane;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) dst[q] = e + q < k ? src[e + q] : (uint16_t)0;
+            }
+        }
+        uint8_t* xst = st + WV * G::WBYTES;
+#pragma unroll
+        for (int u = 0; u < G::XCOPIES; ++u) {
+            const int q0 = wave + WV * u, q = q0 < G::XPIECES ? q0 : G::XPIECES - 1;  // the last piece again
+            constexpr int PR = KC / 256;  // pieces of an activation row
+            const int t = t0 + q / PR < rows ? t0 + q / PR : rows - 1;
+            const uint32_t dst = (uint32_t)((q / PR) * G::XROW + 1024 * (q % PR));
+            if constexpr (VEC) {
+                const uint32_t at = 4u * KC * (uint32_t)sc + 1024u * (uint32_t)(q % PR) + 16u * (uint32_t)lane;
+                lds_dma16(at < 2 * rb ? at : 2 * rb - 16, x + (int64_t)t * k, lds_addr(xst) + dst);
+            } else {
+                const int e = KC * sc + 256 * (q % PR) + 4 * lane;
+                const float* src = x + (int64_t)t * k;
+                float* d = reinterpret_cast<float*>(xst + dst) + 4 * lane;
+#pragma unroll
+                for (int z = 0; z < 4; ++z) d[z] = e + z < k ? src[e + z] : 0.0f;
+            }
+        }
+    };
+    auto cvt = [](uint32_t h) { return BF16 ? __builtin_bit_cast(float, h << 16) : f16_to_f32(h); };
+    // `tail`: a stage that the row may end in; the others run without a branch, so that the LDS
+    // reads of a step are issued under the products of the one before
+    auto stage = [&](auto tail, int s) __attribute__((always_inline)) {
+        const uint8_t* st = lds + (s % NS) * G::STAGE;
+        const uint8_t* ws = st + wave * G::WBYTES + i * G::WPIECE + 4 * b;
+        const uint8_t* xs = st + WV * G::WBYTES + i * G::XROW + 8 * b;
+#pragma unroll
+        for (int m = 0; m < G::MC; ++m) {
+            float2 xb[C];
+#pragma unroll
+            for (int c = 0; c < C; ++c) xb[c] = *reinterpret_cast<const float2*>(xs + 4 * c * G::XROW + 128 * m);
+            float a[R][2];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const uint32_t w = *reinterpret_cast<const uint32_t*>(ws + (r / G::RPC) * 4 * G::WPIECE +
+                                                                      (r % G::RPC) * 2 * KC + 64 * m);
+                a[r][0] = cvt(w & 0xFFFFu);
+                a[r][1] = BF16 ? __builtin_bit_cast(float, w & 0xFFFF0000u) : cvt(w >> 16);
+            }
+            if constexpr (decltype(tail)::value) {  // elements past the row: 0 times -0.0, which no sum sees
+                const int e = KC * s + 32 * m + 2 * b;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    a[r][0] = e < k ? a[r][0] : 0.0f;
+                    a[r][1] = e + 1 < k ? a[r][1] : 0.0f;
+                }
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    xb[c].x = e < k ? xb[c].x : -0.0f;
+                    xb[c].y = e + 1 < k ? xb[c].y : -0.0f;
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    acc[r][c][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r][0], xb[c].x, acc[r][c][0], 0, 0, 0);
+                    acc[r][c][1] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[r][1], xb[c].y, acc[r][c][1], 0, 0, 0);
+                }
+        }
+    };
+    if (ns > 0) {
+        const int whole = k / KC;
+#pragma unroll
+        for (int s = 0; s < NS - 1; ++s) issue(s);
+        for (int s = 0; s < ns; ++s) {
+            // stage s has landed (the NS - 2 after it may fly), the previous one is read out, and the
+            // next copies go into its place
+            wait_vm<VEC ? G::COPIES * (NS - 2) : 0>();
+            lds_barrier();
+            issue(s + NS - 1);
+            if (s < whole)
+                stage(std::false_type{}, s);
+            else
+                stage(std::true_type{}, s);
+        }
+        wait_vm<0>();  // the last (repeated) copies have landed before the workgroup ends
+    }
+    // the halving fold: accumulators 2 b + j and 16 on (block b + 8), 8 on (b + 4), 4 on (b + 2),
+    // 2 on (b + 1), then the lane's own two; block 0 (lanes 0 to 3) ends with the sums
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int t = t0 + 4 * c + i;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float v[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    uint32_t u = f2u(acc[r][c][j][q]);
+                    const auto h16 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+                    u = f2u(u2f(h16[0]) + u2f(h16[1]));
+                    const auto h8 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+                    float f = u2f(h8[0]) + u2f(h8[1]);
+                    f = f + u2f(dpp_u32<0x108>(f2u(f)));  // row_shl:8
+                    f = f + u2f(dpp_u32<0x104>(f2u(f)));  // row_shl:4
+                    v[j] = f;
+                }
+                const int row = row0 + 4 * r + q;
+                if (lane < 4 && t < rows && row < n_out) y[(int64_t)t * n_out + row] = v[0] + v[1];
+            }
+        }
+}
+
+template <int BF16, int VEC, int C, int R, int WV, int KC, int NS>
+static void launch_float(const uint8_t* W, int n_out, int k, const float* x, int rows, float* y, hipStream_t stream,
+                         const uint32_t* active) {
+    using G = GfCfg<C, R, WV, KC, NS>;
+    const int groups = (rows + 4 * C - 1) / (4 * C);
+    int64_t wgs = (n_out + 4 * R * WV - 1) / (4 * R * WV);
+    if (groups > 1) wgs = (wgs + 7) / 8 * 8 * groups;
+    // once per process, thread-safe (a function-local static); a refusal shows as the launch's error
+    static const hipError_t attr = hipFuncSetAttribute((const void*)k_gemv_float<BF16, VEC, C, R, WV, KC, NS>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)G::LDS);
+    (void)attr;
+    hipLaunchKernelGGL((k_gemv_float<BF16, VEC, C, R, WV, KC, NS>), dim3((unsigned)wgs), dim3(64 * WV), G::LDS, stream,
+                       W, n_out, k, x, rows, y, active, groups);
+}
+
+// Workgroups of 64 weight rows (eight wavefronts of eight) from this many of them on, else of
+// sixteen (four wavefronts of four), which spread fewer rows over more CUs: 14336 x 4096 at 2 rows
+// 24.3 us in 224 workgroups against 33.6 in 896, 4096 x 4096 at 24 rows 36 us in 128 against 33.
+constexpr int GF_WIDE_WGS = 129;
+
+// Beyond 16 activation rows, groups of 16 (32 in one workgroup leave one wavefront a SIMD: 32064 x
+// 4096 at 32 rows 192 us against 174).
+template <int BF16>
+static void launch_float_fmt(const uint8_t* W, int n_out, int k, const float* x, int rows, float* y,
+                             hipStream_t stream, const uint32_t* active) {
+    const bool vec = k % 8 == 0 && k <= (1 << 24) && ((uintptr_t)W & 15) == 0 && ((uintptr_t)x & 15) == 0;
+    const bool wide = (int64_t)((n_out + 63) / 64) * ((rows + 15) / 16) >= GF_WIDE_WGS;
+    if (!vec)
+        launch_float<BF16, 0, 4, 1, 4, 512, 2>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 4 && wide)
+        launch_float<BF16, 1, 1, 2, 8, 256, 4>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 4)
+        launch_float<BF16, 1, 1, 1, 4, 512, 4>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 8 && wide)
+        launch_float<BF16, 1, 2, 2, 8, 256, 3>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 8)
+        launch_float<BF16, 1, 2, 1, 4, 512, 4>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 12 && wide)
+        launch_float<BF16, 1, 3, 2, 8, 256, 3>(W, n_out, k, x, rows, y, stream, active);
+    else if (wide)
+        launch_float<BF16, 1, 4, 2, 8, 256, 3>(W, n_out, k, x, rows, y, stream, active);
+    else
+        launch_float<BF16, 1, 4, 1, 4, 512, 3>(W, n_out, k, x, rows, y, stream, active);
+}
+
+void launch_gemv_float(int ty, const uint8_t* W, int n_out, int k, const float* x, int rows, float* y,
+                       hipStream_t stream, const uint32_t* active) {
+    if (ty == T_BF16)
+        launch_float_fmt<1>(W, n_out, k, x, rows, y, stream, active);
+    else
+        launch_float_fmt<0>(W, n_out, k, x, rows, y, stream, active);
+}
+
+}  // namespace syn

@@ -26,10 +26,24 @@ __global__ __launch_bounds__(NORM_THREADS) void k_rms_norm(const float* __restri
     __shared__ float sums[NORM_MAX_BLOCKS];
     const float* xr = x + (int64_t)row * n;
     const int nblocks = (n + 31) / 32;
+    const bool vec = n % 4 == 0 && ((uintptr_t)x & 15) == 0;
     for (int b = threadIdx.x; b < nblocks; b += NORM_THREADS) {
         const int end = (b + 1) * 32 < n ? (b + 1) * 32 : n;
         float acc = 0.0f;
-        for (int i = b * 32; i < end; ++i) acc = acc + xr[i] * xr[i];
+        if (vec && end - b * 32 == 32) {  // the block's 32 values in flight together: one wait, not one a load
+            float4 v[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[q] = reinterpret_cast<const float4*>(xr + b * 32)[q];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                acc = acc + v[q].x * v[q].x;
+                acc = acc + v[q].y * v[q].y;
+                acc = acc + v[q].z * v[q].z;
+                acc = acc + v[q].w * v[q].w;
+            }
+        } else {
+            for (int i = b * 32; i < end; ++i) acc = acc + xr[i] * xr[i];
+        }
         sums[b] = acc;
     }
     __syncthreads();

@@ -392,6 +392,22 @@ def test_float_gemv_equals_oracle(S, ty, rows, n_out, k):
     assert_same(got, o.gemv(ty, w, n_out, k, x, rows, threads=8), f"ty {ty}")
 
 
+@pytest.mark.parametrize("ty", [o.F16, o.BF16])
+@pytest.mark.parametrize("rows,n_out,k,scale", [
+    (4, 17, 512, 1.0), (5, 129, 544, 1.0), (8, 16, 1536, 1.0), (12, 300, 2052, 1.0), (13, 63, 36, 1.0),
+    (16, 1000, 4, 1.0), (17, 200, 260, 1.0), (33, 65, 1028, 1.0), (70, 31, 96, 1.0), (6, 40, 6, 1.0),
+    (2, 16384, 8, 1.0), (9, 16400, 16, 1.0), (31, 16385, 12, 1.0), (3, 100, 640, 3e-41), (5, 50, 96, 1e-36)])
+def test_float_gemv_tiles(S, ty, rows, n_out, k, scale):
+    """The edges of the matrix-core form: activation tiles of 4, their groups (16 and 32 rows), weight
+    tiles, both row widths, chunk and 32-element remainders, subnormal activations and products."""
+    rng = GemvRng(ty * 17 + rows * 5 + k + n_out)
+    w = gemv_weights(rng, ty, n_out, k, o.f16_bits, o.round_bf16)
+    x = (gemv_activations(rng, rows, k) * np.float32(scale)).astype(np.float32)
+    announce(f"float gemv tiles ty={ty} rows={rows} n_out={n_out} k={k}")
+    got = gpu_gemv(S, ty, w, n_out, k, x, rows)
+    assert_same(got, o.gemv(ty, w, n_out, k, x, rows, threads=8), f"ty {ty}")
+
+
 def test_float_gemv_golden_case(S):
     """The pinned output bits of crates/kernels-cpu/src/gemv/tests.rs:726-777 on the device."""
     from test_oracle_pins import PINNED
