@@ -51,9 +51,10 @@ def sources():
     return sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "*.cpp")))
 
 
-# Per-source additions.  gemv_split.hip: the matrix products' results go straight to VGPRs (no
-# accumulation-register reads in the F32 epilogue that follows every product).
-FILE_FLAGS = {"gemv_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# Per-source additions.  gemv_split.hip, gemm_q32.hip: the matrix products' results go straight to
+# VGPRs (no accumulation-register reads in the F32 epilogue that follows every product).
+FILE_FLAGS = {"gemv_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "gemm_q32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _compile(src: str) -> str:

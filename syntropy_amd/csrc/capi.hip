@@ -133,6 +133,28 @@ SYN_EXPORT int syn_act_quantize(int32_t wtype, const float* x, uint32_t rows, ui
     return check_launch(W);
 }
 
+namespace {
+// The products over a matrix in GGUF order from rows quantized by syn_act_quantize: the int8 matrix
+// cores from SOURCE_GEMM_MIN_ROWS rows of Q8_0 or Q4_0 (matrices at even addresses), else the decode
+// kernel, which takes eight rows a launch.  At 8 rows the two are close (6144 x 4096 Q4_0 32 against
+// 37 us, 1024 x 2048 18 against 21; at 4 rows 31 against 24), from 9 the decode kernel takes two
+// launches (16 rows 32 against 70 us, 200 rows 63 against 804).
+constexpr uint32_t SOURCE_GEMM_MIN_ROWS = 8;
+
+void source_products(int32_t wtype, const void* w, uint32_t n_out, uint32_t k_in, const void* ws, uint32_t rows,
+                     float* y, void* stream, const uint32_t* active) {
+    if (rows >= SOURCE_GEMM_MIN_ROWS && aligned(w, 2) && syn::gemm_q32_fits((int)wtype, (int)n_out, (int)k_in, (int)rows)) {
+        const syn::ActLayout L = syn::act_layout(syn::ACT_Q8_0, rows, k_in);
+        const uint8_t* b = (const uint8_t*)ws;
+        syn::launch_gemm_q32((int)wtype, 0, (const uint8_t*)w, (int)n_out, (int)k_in, (const int8_t*)(b + L.codes),
+                             (const float*)(b + L.d), (int)rows, y, (hipStream_t)stream, active);
+        return;
+    }
+    syn::launch_gemv_q(wtype, (const uint8_t*)w, (int)n_out, (int)k_in, (const uint8_t*)ws, (int)rows, y,
+                       (hipStream_t)stream, active);
+}
+}  // namespace
+
 SYN_EXPORT int syn_gemv_quantized(int32_t wtype, const void* w, uint64_t w_bytes, uint32_t n_out,
                                   uint32_t k_in, const void* ws, uint64_t ws_bytes, uint32_t rows,
                                   float* y, void* stream) {
@@ -157,8 +179,7 @@ SYN_EXPORT int syn_gemv_quantized(int32_t wtype, const void* w, uint64_t w_bytes
         syn::launch_gemv_q4k_dec_ws((const uint8_t*)w, (int)n_out, (int)k_in, (const uint8_t*)ws, y,
                                     (hipStream_t)stream);
     else
-        syn::launch_gemv_q(wtype, (const uint8_t*)w, (int)n_out, (int)k_in, (const uint8_t*)ws,
-                           (int)rows, y, (hipStream_t)stream);
+        source_products(wtype, w, n_out, k_in, ws, rows, y, stream, nullptr);
     return check_launch(W);
 }
 
@@ -237,8 +258,7 @@ int syn_gemv_rows(int32_t wtype, const void* w, uint64_t w_bytes, uint32_t n_out
         syn::launch_act_quant(syn::act_kind(wtype), x, rows, k_in, (uint8_t*)ws, (hipStream_t)stream);
         if (int rc = check_launch(W)) return rc;
     }
-    syn::launch_gemv_q(wtype, (const uint8_t*)w, (int)n_out, (int)k_in, (const uint8_t*)ws, (int)rows,
-                       y, (hipStream_t)stream, active);
+    source_products(wtype, w, n_out, k_in, ws, rows, y, stream, active);
     return check_launch(W);
 }
 
@@ -617,7 +637,12 @@ bool split_gemm(int32_t wtype, uint32_t n_out, uint32_t k_in, uint32_t rows) {
     if (wtype != SYN_Q8_0 && wtype != SYN_Q4_0) return false;
     if (rows >= 2 && syn::gemm_q8_staged_fits((int)wtype, (int)n_out, (int)k_in, (int)rows))
         return staged_faster(wtype, n_out, k_in, rows);
-    return wtype == SYN_Q8_0 && rows >= SPLIT_GEMM_MIN_ROWS;
+    if (wtype == SYN_Q8_0) return rows >= SPLIT_GEMM_MIN_ROWS;
+    // Q4_0 rows that are not whole stages: the matrix cores' time at few rows follows the row length
+    // (2.1k values 18 us, 4.1k 29, 14k 85), the decode kernel's the number of eights of rows (1111 x
+    // 2080: 17 us at 16 rows, 30 at 33; 4096 x 4128: 24 and 50; 2000 x 14240: 53 and 112).
+    return rows >= (k_in <= 2048 ? 9u : k_in <= 8192 ? 17u : 33u) &&
+           syn::gemm_q32_fits((int)wtype, (int)n_out, (int)k_in, (int)rows);
 }
 
 // The products over a SPLIT matrix from rows already quantized to Q8_0 blocks in ws.
@@ -1180,12 +1205,22 @@ int moe_grouped_q8_0(const void* gate, const void* up, const void* down, uint64_
     int8_t* hq = (int8_t*)(base + m.hq);
     float* hd = (float*)(base + m.hd);
     syn::launch_moe_pack(ids, ent, (int)n_experts, offsets, slots, err, st, active, (int)top_k, site, report);
-    syn::launch_moe_gather_q8_0(x, slots, ent, (int)top_k, (int)hidden, err, xq, xd, 1, offsets + n_experts, st);
-    syn::launch_moe_q8(0, (const uint8_t*)gate, (const uint8_t*)up, mat, (int)n_experts, (int)inter, (int)hidden,
-                       offsets, slots, err, xq, xd, h, st);
-    syn::launch_moe_gather_q8_0(h, slots, ent, (int)top_k, (int)inter, err, hq, hd, 0, offsets + n_experts, st);
-    syn::launch_moe_q8(1, (const uint8_t*)down, nullptr, mat, (int)n_experts, (int)hidden, (int)inter, offsets,
-                       slots, err, hq, hd, out, st);
+    if (syn::gemm_q32_fits(SYN_Q8_0, (int)inter, (int)hidden, ent) &&
+        syn::gemm_q32_fits(SYN_Q8_0, (int)hidden, (int)inter, ent)) {
+        syn::launch_moe_gather_q8_0(x, nullptr, (int)rows, 1, (int)hidden, err, xq, xd, 0, nullptr, st);
+        syn::launch_moe_q32(0, (const uint8_t*)gate, (const uint8_t*)up, mat, (int)n_experts, (int)inter, (int)hidden,
+                            offsets, slots, err, (int)top_k, (int)rows, ent / (int)n_experts, xq, xd, h, st);
+        syn::launch_moe_gather_q8_0(h, slots, ent, (int)top_k, (int)inter, err, hq, hd, 0, offsets + n_experts, st);
+        syn::launch_moe_q32(1, (const uint8_t*)down, nullptr, mat, (int)n_experts, (int)hidden, (int)inter, offsets,
+                            slots, err, (int)top_k, (int)rows, ent / (int)n_experts, hq, hd, out, st);
+    } else {
+        syn::launch_moe_gather_q8_0(x, slots, ent, (int)top_k, (int)hidden, err, xq, xd, 1, offsets + n_experts, st);
+        syn::launch_moe_q8(0, (const uint8_t*)gate, (const uint8_t*)up, mat, (int)n_experts, (int)inter, (int)hidden,
+                           offsets, slots, err, xq, xd, h, st);
+        syn::launch_moe_gather_q8_0(h, slots, ent, (int)top_k, (int)inter, err, hq, hd, 0, offsets + n_experts, st);
+        syn::launch_moe_q8(1, (const uint8_t*)down, nullptr, mat, (int)n_experts, (int)hidden, (int)inter, offsets,
+                           slots, err, hq, hd, out, st);
+    }
     if (status) {
         hipError_t e = hipMemcpyAsync(status, err, 4, hipMemcpyDeviceToDevice, st);
         if (e != hipSuccess) return fail(SYN_E_DEVICE, "%s: status copy: %s", W, hipGetErrorString(e));

@@ -1050,6 +1050,16 @@ void launch_gemm_q8_split(int ty, const uint8_t* W, int n_out, int k, const uint
     const ActLayout L = act_layout(ACT_Q8_0, (uint64_t)T, (uint64_t)k);
     const int8_t* xq = reinterpret_cast<const int8_t*>(ws + L.codes);
     const float* xd = reinterpret_cast<const float*>(ws + L.d);
+    // gemm_q32.hip: rows that are not whole stages (4096 x 4128 Q8_0 at 256 rows 33 us against 127 for
+    // the register-staged kernel, Q4_0 34 against 344 for the decode kernel eight rows at a time), and
+    // from Q32_MIN_TILES 32 x 32 output tiles on, about one a SIMD (4096 x 14336 Q8_0 at 256 rows,
+    // 1024 tiles: 88 against 99 us; at 128 rows, 512 tiles: 81 against 65)
+    constexpr int64_t Q32_MIN_TILES = 896;
+    if (gemm_q32_fits(ty, n_out, k, T) &&
+        (!gemm_q8_staged_fits(ty, n_out, k, T) || (T > 32 && (int64_t)((n_out + 31) / 32) * ((T + 31) / 32) >= Q32_MIN_TILES))) {
+        launch_gemm_q32(ty, 1, W, n_out, k, xq, xd, T, y, stream, active);
+        return;
+    }
     if (use_splitk(ty, n_out, k, T)) {  // rows of whole 16-block stages, up to 32 tokens
         if (ty == T_Q4_0)
             launch_splitk<T_Q4_0>(W, n_out, k, xq, xd, T, y, stream, active);

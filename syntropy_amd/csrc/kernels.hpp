@@ -57,6 +57,16 @@ void launch_moe_gather_q8_0(const float* x, const uint32_t* slots, int nentries,
 void launch_moe_q8(int mode, const uint8_t* w0, const uint8_t* w1, uint64_t mat_bytes, int n_experts, int n_out,
                    int k, const uint32_t* offsets, const uint32_t* slots, const uint32_t* err, const int8_t* aq,
                    const float* ad, float* y, hipStream_t stream);
+// gemm_q32.hip: Q8_0 / Q4_0 products at many rows on the matrix cores, the matrix in GGUF (split 0) or
+// SPLIT order; activations Q8_0 rows (codes [T][k], scales [T][k / 32])
+bool gemm_q32_fits(int ty, int n_out, int k, int T);
+void launch_gemm_q32(int ty, int split, const uint8_t* W, int n_out, int k, const int8_t* xq, const float* xd, int T,
+                     float* y, hipStream_t stream, const uint32_t* active = nullptr);
+// MoeGrouped's products over Q8_0 experts.  mode 0: gate and up on the tokens' rows (entry i reads
+// row slots[i] / top_k), y[entry] = silu(g) u; mode 1: down on the entries' rows, y[slot]
+void launch_moe_q32(int mode, const uint8_t* w0, const uint8_t* w1, uint64_t mat_bytes, int n_experts, int n_out, int k,
+                    const uint32_t* offsets, const uint32_t* slots, const uint32_t* err, int top_k, int max_entries,
+                    int avg_entries, const int8_t* xq, const float* xd, float* y, hipStream_t stream);
 // gemv_split.hip: Q8_0 / Q4_0 in the SPLIT layout (codes, then scales); activations Q8_0 rows
 void launch_split_repack(int ty, const uint8_t* src, uint8_t* dst, uint64_t bytes, int inverse, hipStream_t stream);
 void launch_gemv_split(int ty, const uint8_t* W, int n_out, int k, const uint8_t* ws, int rows, float* y,

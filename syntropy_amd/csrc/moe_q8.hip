@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256) void k_moe_gather_q8_0(const float* __restrict
     const int sub = threadIdx.x & 7;
     const uint64_t entry = blk / (uint64_t)nb;
     const int b = (int)(blk - entry * (uint64_t)nb);
-    const bool live = entry < (uint64_t)nentries && entry < (uint64_t)*total;  // uniform per block
+    const bool live = entry < (uint64_t)nentries && (!total || entry < (uint64_t)*total);  // uniform per block
     float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
     if (live) {
         const uint64_t row = gather ? slots[entry] / (uint32_t)top_k : entry;

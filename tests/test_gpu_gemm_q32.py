@@ -1,0 +1,111 @@
+"""The Q8_0 / Q4_0 products on the matrix cores (csrc/gemm_q32.hip) at the edges of their tiles, against
+the oracle bit for bit: rows and tokens around 32, 64 and 128, row lengths of whole and partial
+four-block stages, matrices at every even offset of a 16-byte piece, the wide form, infinite and NaN
+scales, and expert lists longer than the launch's grid."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import announce, assert_same, dev, host, require_gpu
+from oracle import oracle as o
+
+pytestmark = pytest.mark.gpu
+BYTES = {o.Q8_0: 34, o.Q4_0: 18}
+
+
+@pytest.fixture(scope="module")
+def S():
+    require_gpu()
+    import syntropy_amd.gemv as S
+    return S
+
+
+def blocks(rs, ty, n_out, k):
+    """Random codes, F16 scales of either sign with biased exponents 3..12."""
+    nb = n_out * k // 32
+    b = rs.integers(0, 256, (nb, BYTES[ty]), dtype=np.uint8)
+    h = (rs.integers(0, 2, nb) << 15) | (rs.integers(3, 13, nb) << 10) | rs.integers(0, 1024, nb)
+    b[:, :2] = h.astype(np.uint16).view(np.uint8).reshape(nb, 2)
+    return b.reshape(-1)
+
+
+def check(S, ty, w, n_out, k, x, rows, what):
+    want = o.gemv(ty, w, n_out, k, x, rows, threads=16)
+    announce(what)
+    W = S.Weights(S.WeightType(ty), dev(w), n_out, k)
+    assert_same(host(S.gemv(W, dev(x), rows)), want, what)
+    assert_same(host(S.gemv(S.repack(W), dev(x), rows)), want, what + " split")
+
+
+@pytest.mark.parametrize("ty", [o.Q8_0, o.Q4_0])
+@pytest.mark.parametrize("rows,n_out,k", [
+    (8, 1, 32), (9, 31, 64), (17, 33, 96), (32, 64, 128), (33, 65, 160), (63, 63, 256), (64, 130, 288),
+    (65, 32, 1056), (130, 97, 416), (40, 3, 2080), (35, 129, 4128), (1, 64, 160), (5, 64, 160)])
+def test_tile_edges(S, ty, rows, n_out, k):
+    rs = np.random.default_rng(rows * 131 + n_out + k)
+    x = rs.standard_normal((rows, k)).astype(np.float32)
+    check(S, ty, blocks(rs, ty, n_out, k), n_out, k, x, rows, f"q32 ty={ty} rows={rows} {n_out}x{k}")
+
+
+@pytest.mark.parametrize("ty", [o.Q8_0, o.Q4_0])
+@pytest.mark.parametrize("rows,n_out,k", [(2100, 2053, 96), (1025, 4099, 160)])
+def test_wide_form(S, ty, rows, n_out, k):
+    """Two token tiles a wavefront, the last of them partial or empty."""
+    rs = np.random.default_rng(rows + k)
+    x = rs.standard_normal((rows, k)).astype(np.float32)
+    check(S, ty, blocks(rs, ty, n_out, k), n_out, k, x, rows, f"q32 wide ty={ty} rows={rows} {n_out}x{k}")
+
+
+@pytest.mark.parametrize("ty", [o.Q8_0, o.Q4_0])
+def test_offsets(S, ty):
+    """GGUF rows from any address: every even offset of a 16-byte piece, and odd ones."""
+    n_out, k, rows = 37, 224, 20
+    rs = np.random.default_rng(5)
+    w, x = blocks(rs, ty, n_out, k), rs.standard_normal((rows, k)).astype(np.float32)
+    want = o.gemv(ty, w, n_out, k, x, rows)
+    for at in (1, 2, 4, 6, 8, 10, 12, 13, 14):
+        buf = torch.zeros(w.size + 32, dtype=torch.uint8, device="cuda")
+        buf[at:at + w.size] = dev(w)
+        announce(f"q32 ty={ty} at {at}")
+        W = S.Weights(S.WeightType(ty), buf[at:at + w.size], n_out, k)
+        assert_same(host(S.gemv(W, dev(x), rows)), want, f"at {at}")
+
+
+@pytest.mark.parametrize("ty", [o.Q8_0, o.Q4_0])
+def test_infinite_and_nan_scales(S, ty):
+    """An infinite weight scale or activation scale (past F16's range), a NaN one, a NaN activation, an
+    all-zero row: the reference's infinities and NaNs, and every other output as it is."""
+    n_out, k, rows = 70, 192, 40
+    rs = np.random.default_rng(11)
+    w = blocks(rs, ty, n_out, k).reshape(n_out, k // 32, BYTES[ty])
+    w[3, 2, :2] = np.array([0x7C00], np.uint16).view(np.uint8)
+    w[40, 0, :2] = np.array([0xFC00], np.uint16).view(np.uint8)
+    w[66, 5, :2] = np.array([0x7E00], np.uint16).view(np.uint8)
+    w[50, 1, :2] = 0
+    x = rs.standard_normal((rows, k)).astype(np.float32)
+    x[2, 33:64] *= 3e8   # the block's scale rounds to an infinity
+    x[34, 70] = np.nan
+    x[35, 5] = np.inf
+    x[36] = 0.0
+    x[37] *= 1e-6        # subnormal scales
+    check(S, ty, w.reshape(-1), n_out, k, x, rows, f"q32 ty={ty} infinite scales")
+
+
+@pytest.mark.parametrize("E,top_k,hidden,inter,rows,popular", [
+    (4, 1, 160, 96, 300, 290),    # one expert's entries beyond the grid's tiles
+    (3, 2, 64, 224, 70, 65), (6, 2, 288, 64, 90, 0), (16, 2, 96, 160, 33, 20), (1, 1, 32, 32, 129, 129)])
+def test_experts(S, E, top_k, hidden, inter, rows, popular):
+    import syntropy_amd.moe as M
+    rs = np.random.default_rng(E * 7 + rows)
+    gate, up, down = (blocks(rs, o.Q8_0, E * n, k) for n, k in ((inter, hidden), (inter, hidden), (hidden, inter)))
+    up.reshape(E, inter, hidden // 32, 34)[0, 5, 0, :2] = np.array([0x7C00], np.uint16).view(np.uint8)
+    x = rs.standard_normal((rows, hidden)).astype(np.float32)
+    ids = np.stack([rs.permutation(E)[:top_k] for _ in range(rows)]).astype(np.int32)
+    ids[:popular, 0] = 0
+    if top_k > 1:
+        ids[:popular, 1:] = 1 + np.arange(top_k - 1)
+    want = o.moe_grouped(o.Q8_0, o.Q8_0, E, top_k, hidden, inter, gate, up, down, x, ids, threads=8)
+    announce(f"q32 experts E={E} k={top_k} {hidden} {inter} rows={rows}")
+    ex = M.Experts(M.WeightType.Q8_0, dev(gate), dev(up), dev(down))
+    got = M.moe_grouped(M.MoeShape(E, top_k, hidden, inter), ex, dev(x), dev(ids))
+    assert_same(host(got), want, "experts")
