@@ -27,11 +27,15 @@
 // the codes of four consecutive bytes, low nibbles then high: k_gemm_act writes the activations
 // in the same order.
 //
-// Tiling.  A workgroup computes 64 tokens x 256 rows; each of its 8 wavefronts 64 tokens x 32
-// rows as 4 x 2 tiles of 16 x 16 (two wavefronts per SIMD hide each other's LDS and matrix-core
-// latencies), so each A operand serves two row tiles and each B operand four token tiles.  Per super-block the weight rows (144 bytes each), the 64 tokens' codes and their
-// sums, scales and X stream from global memory into LDS with global_load_lds_dwordx4 (no
-// registers held while they fly), one stage ahead, in a ring of two 72 KB stages.
+// Tiling.  A wavefront computes 16 MT tokens x 16 NT rows as MT x NT tiles of 16 x 16, a workgroup four
+// of them, one below the other.  The tokens' codes, sums, scales and X stream into LDS by
+// global_load_lds_dwordx4 (no registers held while they fly); a row's weights serve one wavefront and
+// go straight to its registers.  What bounds it: the vector ALU and the matrix cores, whose times add
+// (per super-block and 64 tokens x 32 rows about 1150 cycles of matrix products, 560 of the fold's
+// seven F32 operations an output, 700 of building B), then one wavefront's issue rate where a shape
+// gives a SIMD only one.  14336 x 4096, X8, 2048 rows: 388 us (620 TFLOP/s) against 491 for workgroups of
+// eight 64 x 32 wavefronts, one a CU, whose weights went through LDS; 4096 x 14336 at 64 rows 63 us
+// against 220.
 #include <type_traits>
 #include "common.hpp"
 #include "kernels.hpp"
@@ -169,21 +173,27 @@ void launch_gemm_act(const float* x, int T, int k, GemmAct a, hipStream_t stream
 // The GEMM
 // ============================================================================================
 
-constexpr int GM_TT = 64;                           // tokens per workgroup
-constexpr int GM_WAVES = 8;                         // wavefronts per workgroup
-constexpr int GM_NT = 2;                            // 16-row tiles per wavefront
-constexpr int GM_MT = 4;                            // 16-token tiles per wavefront
-constexpr int GM_ROWS = GM_WAVES * 16 * GM_NT;      // rows per workgroup
-constexpr int GM_WB = GM_ROWS * 144;                // weight bytes per stage
-constexpr int GM_AB = GM_TT * 512;                  // code bytes per stage
-constexpr int GM_TB = GM_TT * GM_TAIL_ROW;          // s2 | dx | X bytes per stage
-constexpr int GM_WSLOT = GM_WB / 1024;              // wavefront loads (64 x 16 bytes) of each part
-constexpr int GM_ASLOT = GM_AB / 1024;
-constexpr int GM_TSLOT = (GM_TB + 1023) / 1024;
-constexpr int GM_WPW = (GM_WSLOT + GM_WAVES - 1) / GM_WAVES;  // weight slots per wavefront (at most)
-constexpr int GM_PER_WAVE = GM_WPW + GM_ASLOT / GM_WAVES + 1;
-static_assert(GM_ASLOT % GM_WAVES == 0 && GM_TSLOT <= GM_WAVES, "slot split");
-static_assert(GM_WB % 1024 == 0 && GM_AB % 1024 == 0, "wavefront-sized weight and code parts");
+constexpr int GM_WAVES = 4;                         // wavefronts per workgroup
+
+// NT: 16-row tiles of a wavefront.
+constexpr int gemm_rows(int nt) { return GM_WAVES * 16 * nt; }  // rows per workgroup
+
+// MT: 16-token tiles, of a workgroup as of each of its wavefronts.  A stage is half a super-block of
+// the tokens' codes: k steps 4 h .. 4 h + 3 of the eight.
+template <int MT>
+struct GmCfg {
+    static constexpr int TT = 16 * MT;              // tokens
+    static constexpr int AB = TT * 256;             // token code bytes per stage
+    static constexpr int TB = TT * GM_TAIL_ROW;     // s2 | dx | X bytes per super-block
+    // HALVES: two stages and one super-block's tail; else two super-blocks with theirs
+    template <bool HALVES>
+    static constexpr int TAIL = (HALVES ? 2 : 4) * AB;
+    template <bool HALVES>
+    static constexpr int LDS = TAIL<HALVES> + (HALVES ? 1 : 2) * TB;
+    static constexpr int APW = AB / 1024 / GM_WAVES;  // a wavefront's loads (64 x 16 bytes) of a stage
+    static constexpr int TPW = (TB / 16 + 64 * GM_WAVES - 1) / (64 * GM_WAVES);
+    static_assert(AB % (1024 * GM_WAVES) == 0, "stage copies split evenly");
+};
 
 struct GemmArgs {
     const uint8_t* W;
@@ -193,66 +203,93 @@ struct GemmArgs {
     float* y;
     int N, T, nb, tpad;
     uint32_t rb;  // weight row bytes
+    int xcd_tokens;  // token tiles an XCD takes (a 1-D grid), or 0: blockIdx.x, blockIdx.y the row and token tiles
     const uint32_t* active;  // a step descriptor's rows_active, or null
 };
 
-// The lane's 32-bit offsets of its loads of one stage, relative to the part's base of the
-// super-block (weights: W + 144 b; codes: codes + (b tpad + t0) 512; tail: tail + b tpad 40).
-struct GemmSlots {
-    uint32_t woff[GM_WPW];
-    uint32_t toff;
-    int nw, nt;     // weight and tail slots of this wavefront (uniform)
-    bool ton;       // this lane's tail chunk exists
+// A super-block of the lane's rows (16 nt + lane % 16 of the wavefront's 32): the row header and, of
+// lane group p, bytes 32 p .. + 31 of the codes.  A row's weights serve one wavefront, so they go
+// straight to its registers, half a super-block ahead.
+template <int NT>
+struct GemmW {
+    v4u hdr[NT], q[NT][2];
 };
 
-SYN_DEV GemmSlots gemm_slots(const GemmArgs& g, int wave, int lane, int n0, int t0) {
-    GemmSlots s;
-    s.nw = 0;
+SYN_DEV uint32_t gemm_chunk_step(int layout) { return layout == LAYOUT_X8 ? 128u : 16u; }
+SYN_DEV uint32_t gemm_row_offset(int layout, uint32_t r, uint32_t rb) {
+    return layout == LAYOUT_TILE64 ? (uint32_t)tile64_row_offset(r, rb) : r * rb;
+}
+
+// wb: the super-block of the matrix's row 0; off: the lane's rows from there; qoff: its chunks 1 + 2 p.
+template <int NT>
+SYN_DEV GemmW<NT> gemm_weights(const uint8_t* wb, const uint32_t (&off)[NT], const uint32_t (&qoff)[NT],
+                               uint32_t chunk_step) {
+    GemmW<NT> w;
 #pragma unroll
-    for (int u = 0; u < GM_WPW; ++u) {
-        const int gs = wave + GM_WAVES * u;
-        const int ci = 64 * gs + lane, row = ci / 9, part = ci - 9 * (ci / 9);
-        const int r = n0 + row < g.N ? n0 + row : g.N - 1;
-        // chunk `part` of the row's block: 16 bytes on in GGUF order and TILE64, 128 (a run's chunk
-        // row) in X8
-        s.woff[u] = g.layout == LAYOUT_TILE64 ? (uint32_t)tile64_row_offset((uint32_t)r, g.rb) + 16u * (uint32_t)part
-                                               : (uint32_t)r * g.rb + (g.layout == LAYOUT_X8 ? 128u : 16u) * (uint32_t)part;
-        if (gs < GM_WSLOT) s.nw = u + 1;
+    for (int nt = 0; nt < NT; ++nt) {
+        w.hdr[nt] = *reinterpret_cast<const v4u*>(wb + off[nt]);
+        w.q[nt][0] = *reinterpret_cast<const v4u*>(wb + qoff[nt]);
+        w.q[nt][1] = *reinterpret_cast<const v4u*>(wb + chunk_step + qoff[nt]);
     }
-    // tail slot: wave w takes tail part w if it exists
-    s.nt = wave < GM_TSLOT ? 1 : 0;
-    const int ti = 64 * wave + lane;
-    s.ton = s.nt && ti < GM_TB / 16;
-    if (ti < GM_TT * 2)
-        s.toff = (uint32_t)t0 * 32u + 16u * (uint32_t)ti;
-    else if (ti < GM_TT * 2 + GM_TT / 4)
-        s.toff = (uint32_t)g.tpad * 32u + (uint32_t)t0 * 4u + 16u * (uint32_t)(ti - GM_TT * 2);
-    else
-        s.toff = (uint32_t)g.tpad * 36u + (uint32_t)t0 * 4u + 16u * (uint32_t)(ti - GM_TT * 2 - GM_TT / 4);
+    return w;
+}
+
+// The source chunk of token copy u (half 0; half 1 has bit 2 flipped) for a token whose row is skewed
+// by `skew`: line 4 u + lane / 16 holds logical chunk (p, s) at position (4 p + s) ^ (line & 15), so
+// that the 16 lines of a read touch 16 different 16-byte bank groups.
+SYN_DEV uint32_t gemm_achunk(int u, int lane, uint32_t skew) {
+    const int slot = (lane & 15) ^ ((4 * u + (lane >> 4)) & 15);
+    return (uint32_t)(8 * (slot >> 2) + (slot & 3)) ^ (skew & 15u);
+}
+
+// The lane's 32-bit offsets of its copies, relative to the part's base of the super-block: token codes
+// (of copy 0: 16 tokens on for each further one; half 1 has bit 6 flipped) and tail.
+template <int MT>
+struct GemmSlots {
+    uint32_t aoff;
+    int left;  // positions that exist from t0 on (a multiple of 64); a tile past them re-reads the last
+    uint32_t toff[GmCfg<MT>::TPW];
+};
+
+template <int MT>
+SYN_DEV GemmSlots<MT> gemm_slots(int tpad, int wave, int lane, int t0) {
+    using C = GmCfg<MT>;
+    GemmSlots<MT> s;
+    const int left = s.left = tpad - t0;
+    const int t = 4 * wave + (lane >> 4);  // of copy 0
+    s.aoff = (uint32_t)t * 512u + 16u * gemm_achunk(wave, lane, (uint32_t)t);
+#pragma unroll
+    for (int i = 0; i < C::TPW; ++i) {
+        // tokens' s2 (two pieces a token), then scales and code sums (a piece for four tokens)
+        const int ti = 64 * (wave + GM_WAVES * i) + lane;
+        const int part = ti < C::TT * 2 ? 0 : ti < C::TT * 2 + C::TT / 4 ? 1 : 2;
+        const int at = part == 0 ? ti : ti - C::TT * 2 - (part - 1) * (C::TT / 4);
+        const int end = part == 0 ? left * 2 : left / 4;
+        s.toff[i] = (uint32_t)tpad * (part == 0 ? 0u : 28u + 4u * (uint32_t)part) + (uint32_t)t0 * (part == 0 ? 32u : 4u) +
+                    16u * (uint32_t)(at < end ? at : end - 1);
+    }
     return s;
 }
 
-
-// Issues the wavefront's loads of super-block b: weights and codes into `stage`, the tail into
-// `tail`.  Slot order: weight parts wave, wave + 8, ..; code parts wave, wave + 8, ..; tail part
-// `wave`.
-SYN_DEV void gemm_issue(const GemmArgs& g, const GemmSlots& s, int wave, int lane, int b, int t0,
+// Issues the wavefront's copies of half H of the tokens' super-block at `ab` to `stage`; half 1 brings
+// the tail.
+template <int MT, int H>
+SYN_DEV void gemm_issue(const GemmSlots<MT>& s, const uint8_t* ab, const uint8_t* tb, int wave, int lane,
                         uint8_t* stage, uint8_t* tail) {
-    // super-block b of row 0: in X8 block b sits in run b / 8 at position b % 8
-    const uint8_t* wb = g.layout == LAYOUT_X8 ? g.W + 1152 * (size_t)(b >> 3) + 16 * (size_t)(b & 7)
-                                                  : g.W + 144 * (size_t)b;
-    const uint8_t* ab = g.codes + ((size_t)b * g.tpad + t0) * 512;
-    const uint8_t* tb = g.tail + (size_t)b * g.tpad * GM_TAIL_ROW;
-    const uint32_t st = lds_addr(stage);
+    using C = GmCfg<MT>;
 #pragma unroll
-    for (int u = 0; u < GM_WPW; ++u)
-        if (u < s.nw) lds_dma16(s.woff[u], wb, st + 1024u * (uint32_t)(wave + GM_WAVES * u));
-#pragma unroll
-    for (int u = 0; u < GM_ASLOT / GM_WAVES; ++u) {
-        const int gs = wave + GM_WAVES * u;
-        lds_dma16(16u * (uint32_t)lane, ab + 1024 * gs, st + (uint32_t)GM_WB + 1024u * (uint32_t)gs);
+    for (int i = 0; i < C::APW; ++i) {
+        static_assert(GM_WAVES == 4, "16 tokens a round of copies");
+        lds_dma16(s.aoff ^ (64u * H), ab + 512u * (uint32_t)(16 * i < s.left ? 16 * i : s.left - 16),
+                  lds_addr(stage) + 1024u * (uint32_t)(wave + GM_WAVES * i));
     }
-    if (s.ton) lds_dma16(s.toff, tb, lds_addr(tail) + 1024u * (uint32_t)wave);
+    if constexpr (H == 1) {
+#pragma unroll
+        for (int i = 0; i < C::TPW; ++i) {
+            const int u = wave + GM_WAVES * i;
+            if (64 * u + lane < C::TB / 16) lds_dma16(s.toff[i], tb, lds_addr(tail) + 1024u * (uint32_t)u);
+        }
+    }
 }
 
 // The F16 pair (1024 + 16 q0, 1024 + 16 q1) etc. from the nibbles under `mask`.
@@ -264,97 +301,105 @@ SYN_DEV h2 magic_pair(uint32_t v, uint32_t mask) {
 
 SYN_DEV h2 bcast(_Float16 v) { return h2{v, v}; }
 
-// What the fold of a super-block needs from its row headers: d, dmin and the S2 operand.
+// What a super-block's products and fold need from its row headers: the pairs (sc, -(1024 sc + 512)) of
+// sub-block 2p and (sc/16, -(64 sc + 512)) of 2p + 1, d, dmin and the minimums.
+template <int NT>
 struct GemmHdr {
-    float dd[GM_NT], dm[GM_NT];
-    v8h bm[GM_NT];
+    h2 ka[NT], kb[NT];
+    float dd[NT], dm[NT];
+    uint32_t mn[NT][2];  // m_0..3, m_4..7
 };
 
-// The matrix-core part of one super-block of the wavefront's 64 tokens x 32 rows, from the
-// weights and codes of the stage in LDS: dacc = S1 - 512 X exactly, and the row headers.  Only
-// the first NMT 16-token tiles are computed (a tile of fewer entries leaves the rest empty).
-template <int NMT>
-SYN_DEV void gemm_mfma(const uint8_t* st, int wave, int lane, v4f (&dacc)[GM_MT][GM_NT], GemmHdr& h) {
-    const int c = lane & 15, p = lane >> 4;
-    const uint8_t* wt = st + (16 * GM_NT * wave) * 144;
-    const uint8_t* at = st + GM_WB;
-    float (&dd)[GM_NT] = h.dd;
-    float (&dm)[GM_NT] = h.dm;
-    v8h (&bm)[GM_NT] = h.bm;
-    h2 ka[GM_NT], kb[GM_NT];  // (sc, -(1024 sc + 512)) of sub-block 2p, (sc/16, -(64 sc + 512)) of 2p + 1
+template <int NT>
+SYN_DEV void gemm_header(const GemmW<NT>& w, int p, GemmHdr<NT>& h) {
 #pragma unroll
-    for (int nt = 0; nt < GM_NT; ++nt) {
-        const v4u hdr = *reinterpret_cast<const v4u*>(wt + (16 * nt + c) * 144);
-        dd[nt] = f16_to_f32(hdr.x);
-        dm[nt] = f16_to_f32(hdr.x >> 16);
+    for (int nt = 0; nt < NT; ++nt) {
+        const v4u hdr = w.hdr[nt];
+        h.dd[nt] = f16_to_f32(hdr.x);
+        h.dm[nt] = f16_to_f32(hdr.x >> 16);
         // get_scale_min_k4 (gemv.rs:528-537) on packed bytes
         const uint32_t w0 = hdr.y, w1 = hdr.z, w2 = hdr.w;
         const uint32_t sc_lo = w0 & 0x3F3F3F3Fu;                                 // sc_0..3
         const uint32_t sc_hi = (w2 & 0x0F0F0F0Fu) | ((w0 >> 2) & 0x30303030u);   // sc_4..7
-        const uint32_t mn_lo = w1 & 0x3F3F3F3Fu;                                 // m_0..3
-        const uint32_t mn_hi = ((w2 >> 4) & 0x0F0F0F0Fu) | ((w1 >> 2) & 0x30303030u);  // m_4..7
+        h.mn[nt][0] = w1 & 0x3F3F3F3Fu;                                          // m_0..3
+        h.mn[nt][1] = ((w2 >> 4) & 0x0F0F0F0Fu) | ((w1 >> 2) & 0x30303030u);     // m_4..7
         // this lane group's sub-blocks: 2p (low nibbles) and 2p + 1 (high nibbles)
         const uint32_t scw = p < 2 ? sc_lo : sc_hi;
         const int sa = (int)((scw >> (16 * (p & 1))) & 0xFFu), sb = (int)((scw >> (16 * (p & 1) + 8)) & 0xFFu);
         const float fa = (float)sa, fb = (float)sb;
-        ka[nt] = h2{(_Float16)fa, (_Float16)(-(1024.0f * fa + 512.0f))};
-        kb[nt] = h2{(_Float16)(fb * 0.0625f), (_Float16)(-(64.0f * fb + 512.0f))};
-        // S2 operand: m_0..m_7 in lane groups 0 and 1 (against l_j and 64 h_j), zero in 2 and 3
-        const _Float16 on = p < 2 ? (_Float16)1.0f : (_Float16)0.0f;
-        const h2 k1 = bcast(on), k0 = bcast((_Float16)(-1024.0f) * on);
-        // bytes b0, b1 of a word into the low bits of two halves
-        const h2 m01 = __builtin_elementwise_fma(__builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, mn_lo, 0x0c010c00u) | 0x64006400u), k1, k0);
-        const h2 m23 = __builtin_elementwise_fma(__builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, mn_lo, 0x0c030c02u) | 0x64006400u), k1, k0);
-        const h2 m45 = __builtin_elementwise_fma(__builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, mn_hi, 0x0c010c00u) | 0x64006400u), k1, k0);
-        const h2 m67 = __builtin_elementwise_fma(__builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, mn_hi, 0x0c030c02u) | 0x64006400u), k1, k0);
-        bm[nt] = v8h{m01.x, m01.y, m23.x, m23.y, m45.x, m45.y, m67.x, m67.y};
+        h.ka[nt] = h2{(_Float16)fa, (_Float16)(-(1024.0f * fa + 512.0f))};
+        h.kb[nt] = h2{(_Float16)(fb * 0.0625f), (_Float16)(-(64.0f * fb + 512.0f))};
     }
+}
 
+// The S2 operand: m_0..m_7 in lane groups 0 and 1 (against l_j and 64 h_j), zero in 2 and 3.
+SYN_DEV v8h gemm_mins(const uint32_t (&mn)[2], int p) {
+    const _Float16 on = p < 2 ? (_Float16)1.0f : (_Float16)0.0f;
+    const h2 k1 = bcast(on), k0 = bcast((_Float16)(-1024.0f) * on);
+    h2 m[4];
 #pragma unroll
-    for (int mt = 0; mt < NMT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < GM_NT; ++nt) dacc[mt][nt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < 4; ++i)  // bytes 2 i, 2 i + 1 into the low bits of two halves
+        m[i] = __builtin_elementwise_fma(
+            __builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, mn[i >> 1], i & 1 ? 0x0c030c02u : 0x0c010c00u) | 0x64006400u), k1, k0);
+    return v8h{m[0].x, m[0].y, m[1].x, m[1].y, m[2].x, m[2].y, m[3].x, m[3].y};
+}
 
+// The matrix-core part of one stage of the wavefront's tokens x 32 rows: dacc = S1 - 512 X exactly
+// once both halves have run (half 0 starts it).  Only the first NMT 16-token tiles are computed (a
+// tile of fewer entries leaves the rest empty).
+template <int MT, int NMT, int H, int NT>
+SYN_DEV void gemm_mfma(const uint8_t* st, const GemmW<NT>& w, int lane, v4f (&dacc)[MT][NT], const GemmHdr<NT>& h) {
+    const int c = lane & 15, p = lane >> 4;
+    const uint8_t* at = st + c * 256;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        v8h bq[GM_NT];
+    for (int s = 0; s < 4; ++s) {
+        v8h bq[NT];
 #pragma unroll
-        for (int nt = 0; nt < GM_NT; ++nt) {
-            // bytes 32p + 4s .. +3 of the row's codes: sub-block 2p (low) and 2p + 1 (high)
-            const uint32_t v = *reinterpret_cast<const uint32_t*>(wt + (16 * nt + c) * 144 + 16 + 32 * p + 4 * s);
+        for (int nt = 0; nt < NT; ++nt) {
+            uint32_t v = w.q[nt][H][s];  // sub-block 2p (low nibbles) and 2p + 1 (high)
+            // keeps a step's operands from being made before it (and spilling)
+            asm volatile("" : "+v"(v) : : "memory");
             // (b0, b2) low nibbles, (b1, b3) low, (b0, b2) high, (b1, b3) high
-            const h2 y3 = __builtin_elementwise_fma(magic_pair(v, 0x000F000Fu), bcast(ka[nt].x), bcast(ka[nt].y));
-            const h2 y2 = __builtin_elementwise_fma(magic_pair(v >> 8, 0x000F000Fu), bcast(ka[nt].x), bcast(ka[nt].y));
-            const h2 y1 = __builtin_elementwise_fma(magic_pair(v, 0x00F000F0u), bcast(kb[nt].x), bcast(kb[nt].y));
-            const h2 y4 = __builtin_elementwise_fma(magic_pair(v >> 8, 0x00F000F0u), bcast(kb[nt].x), bcast(kb[nt].y));
+            const h2 y3 = __builtin_elementwise_fma(magic_pair(v, 0x000F000Fu), bcast(h.ka[nt].x), bcast(h.ka[nt].y));
+            const h2 y2 = __builtin_elementwise_fma(magic_pair(v >> 8, 0x000F000Fu), bcast(h.ka[nt].x), bcast(h.ka[nt].y));
+            const h2 y1 = __builtin_elementwise_fma(magic_pair(v, 0x00F000F0u), bcast(h.kb[nt].x), bcast(h.kb[nt].y));
+            const h2 y4 = __builtin_elementwise_fma(magic_pair(v >> 8, 0x00F000F0u), bcast(h.kb[nt].x), bcast(h.kb[nt].y));
             bq[nt] = v8h{y3.x, y3.y, y2.x, y2.y, y1.x, y1.y, y4.x, y4.y};
         }
 #pragma unroll
         for (int mt = 0; mt < NMT; ++mt) {
-            const int t = 16 * mt + c;
-            const v8h a = *reinterpret_cast<const v8h*>(at + t * 512 + (((8 * p + s) ^ c) << 4));
+            const v8h a = *reinterpret_cast<const v8h*>(at + 16 * mt * 256 + (((4 * p + s) ^ c) << 4));
 #pragma unroll
-            for (int nt = 0; nt < GM_NT; ++nt)
-                dacc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq[nt], dacc[mt][nt], 0, 0, 0);
+            for (int nt = 0; nt < NT; ++nt)
+                dacc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    a, bq[nt], H == 0 && s == 0 ? v4f{0.0f, 0.0f, 0.0f, 0.0f} : dacc[mt][nt], 0, 0, 0);
+            if (mt % 4 == 3) {  // four tiles' operands at a time
+                asm volatile("" : : : "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
     }
 }
 
 // S2 from the tail's code sums, then the super-block's terms folded into the accumulators in
 // the reference's rounding order.
-template <int NMT>
-SYN_DEV void gemm_fold(const uint8_t* tl, int lane, const v4f (&dacc)[GM_MT][GM_NT], const GemmHdr& h,
-                       v4f (&acc)[GM_MT][GM_NT]) {
+template <int MT, int NMT, int NT>
+SYN_DEV void gemm_fold(const uint8_t* tl, int lane, const v4f (&dacc)[MT][NT], const GemmHdr<NT>& h,
+                       v4f (&acc)[MT][NT]) {
+    constexpr int TT = 16 * MT;
     const int c = lane & 15, p = lane >> 4;
     const v8h zero8 = {};
+    v8h bm[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) bm[nt] = gemm_mins(h.mn[nt], p);
 #pragma unroll
     for (int mt = 0; mt < NMT; ++mt) {
         const v8h as = p < 2 ? *reinterpret_cast<const v8h*>(tl + (16 * mt + c) * 32 + 16 * p) : zero8;
-        const v4f dx = *reinterpret_cast<const v4f*>(tl + GM_TT * 32 + (16 * mt + 4 * p) * 4);
-        const v4f xs = *reinterpret_cast<const v4f*>(tl + GM_TT * 36 + (16 * mt + 4 * p) * 4);
+        const v4f dx = *reinterpret_cast<const v4f*>(tl + TT * 32 + (16 * mt + 4 * p) * 4);
+        const v4f xs = *reinterpret_cast<const v4f*>(tl + TT * 36 + (16 * mt + 4 * p) * 4);
 #pragma unroll
-        for (int nt = 0; nt < GM_NT; ++nt) {
-            const v4f s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, h.bm[nt], v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        for (int nt = 0; nt < NT; ++nt) {
+            const v4f s2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, bm[nt], v4f{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float s1 = __builtin_fmaf(512.0f, xs[i], dacc[mt][nt][i]);  // fl(S1), exact operands
@@ -363,103 +408,114 @@ SYN_DEV void gemm_fold(const uint8_t* tl, int lane, const v4f (&dacc)[GM_MT][GM_
                 acc[mt][nt][i] = acc[mt][nt][i] + (a1 - a2);
             }
         }
+        asm volatile("" : "+v"(acc[mt][0]), "+v"(acc[mt][NT - 1]) : : "memory");  // as above: a tile's operands at a time
     }
 }
 
-// The GEMMs' LDS: two stages of weights and codes, then a three-slot ring of tails, so that
-// super-block b's fold can run after b + 1's matrix products (its weights and codes are
-// overwritten by then; its tail is not until b + 3 is issued).
-constexpr int GM_WA = GM_WB + GM_AB;
-constexpr int GM_LOOP_LDS = 2 * GM_WA + 3 * GM_TB;
-static_assert(GM_WA % 16 == 0 && GM_TB % 16 == 0 && GM_LOOP_LDS <= 160 * 1024, "GEMM LDS");
-
-// The super-block loop of both GEMM kernels.  `issue(b, stage, tail)` issues the wavefront's
-// loads of super-block b.  Super-block b's products run first, then b - 1's fold (independent
-// work the wavefront can issue between the products), with the two sets of exact sums
-// alternating by parity.  Super-block 0 has no fold before it, so it is peeled: the loop's
-// products and fold are one straight run of code the scheduler can interleave.  Two schedules
-// of the loads, each a super-block ahead of the products:
-//   AHEAD: two barriers a super-block; once every wavefront has left b's stage, b + 2's loads go
-//     to it at the end of b's step, before the wait for b + 1's, so both may be in flight (the
-//     dense GEMM: 425-434 against 438-444 us a launch at 2048 tokens);
-//   otherwise one barrier a super-block; once every wavefront's loads of b have landed and every
-//     wavefront has left b - 1's products and b - 2's fold, b + 1's loads go to b - 1's stage
-//     and b - 2's tail slot (the MoE layer at 2048 tokens: 1.56 against 1.60 ms).
-// On return every wavefront is done with the two stages (the caller may reuse them); the tail
-// ring may still be read.
-template <int NMT, bool AHEAD, class Issue>
-SYN_DEV void gemm_loop(int nb, int live, uint8_t* smem, int wave, int lane, Issue&& issue,
-                       v4f (&acc)[GM_MT][GM_NT]) {
-    uint8_t* tails = smem + 2 * GM_WA;
-    issue(0, smem, tails);
-    if (AHEAD && nb > 1) issue(1, smem + GM_WA, tails + GM_TB);
-    v4f d0[GM_MT][GM_NT], d1[GM_MT][GM_NT];
-    GemmHdr h0, h1;
-    int slot = 0;  // tail ring slot of b
-    auto step = [&](auto fold, int b, v4f (&dc)[GM_MT][GM_NT], GemmHdr& hc, const v4f (&dp)[GM_MT][GM_NT],
-                    const GemmHdr& hp) __attribute__((always_inline)) {
-        const int prev = slot == 0 ? 2 : slot - 1;  // the slot of b - 1 (b + 2's after the fold)
-        const int next = slot == 2 ? 0 : slot + 1;  // the slot of b + 1 (b - 2's)
-        if constexpr (AHEAD) {
-            wait_vm_n<GM_PER_WAVE>(b + 1 < nb ? live : 0);  // at most b + 1's loads in flight
-        } else {
-            wait_vm<0>();  // b's loads, the only ones in flight
-        }
+// The stage loop of both GEMM kernels.  `issue(half, b, stage, tail)` issues the wavefront's copies of a
+// half of super-block b, `weights(b)` loads its rows.  HALVES: one barrier a half; once every
+// wavefront's copies of a half have landed and every wavefront has left the half before, the next
+// half's copies go to that one's place (the tail, which comes with half 1, after the fold before).
+// Otherwise the same with whole super-blocks: twice the LDS, half the barriers, and a super-block's
+// time for the copies to land, which is what counts where a SIMD holds few wavefronts.  On return
+// the LDS may still be read.
+template <bool HALVES, int MT, int NMT, int NT, class Issue, class Weights>
+SYN_DEV void gemm_loop(int nb, uint8_t* smem, int lane, Issue&& issue, Weights&& weights, v4f (&acc)[MT][NT]) {
+    using C = GmCfg<MT>;
+    std::integral_constant<int, 0> h0;
+    std::integral_constant<int, 1> h1;
+    uint8_t* tails = smem + C::template TAIL<HALVES>;
+    issue(h0, 0, smem, tails);
+    if (!HALVES) issue(h1, 0, smem + C::AB, tails);
+    GemmW<NT> next = weights(0);
+    for (int b = 0; b < nb; ++b) {
+        v4f d[MT][NT];
+        GemmHdr<NT> h;
+        const int buf = HALVES ? 0 : b & 1;
+        uint8_t *st = smem + buf * 2 * C::AB, *tl = tails + buf * C::TB;
+        wait_vm<0>();
         lds_barrier();
-        if (!AHEAD && b + 1 < nb) issue(b + 1, smem + ((b + 1) & 1) * GM_WA, tails + next * GM_TB);
-        gemm_mfma<NMT>(smem + (b & 1) * GM_WA, wave, lane, dc, hc);
-        if constexpr (decltype(fold)::value) {
-            gemm_fold<NMT>(tails + prev * GM_TB, lane, dp, hp, acc);
+        const GemmW<NT> w = next;
+        if constexpr (HALVES) {
+            issue(h1, b, st + C::AB, tl);
+        } else if (b + 1 < nb) {
+            uint8_t *sn = smem + (buf ^ 1) * 2 * C::AB, *tn = tails + (buf ^ 1) * C::TB;
+            issue(h0, b + 1, sn, tn);
+            issue(h1, b + 1, sn + C::AB, tn);
+            next = weights(b + 1);
         }
-        if constexpr (AHEAD) {
+        gemm_header(w, lane >> 4, h);
+        gemm_mfma<MT, NMT, 0>(st, w, lane, d, h);
+        if constexpr (HALVES) {
+            wait_vm<0>();
             lds_barrier();
-            if (b + 2 < nb) issue(b + 2, smem + (b & 1) * GM_WA, tails + prev * GM_TB);
+            if (b + 1 < nb) {
+                issue(h0, b + 1, st, tl);
+                next = weights(b + 1);
+            }
         }
-        slot = next;
-    };
-    step(std::false_type{}, 0, d0, h0, d1, h1);
-    for (int b = 1; b < nb; b += 2) {
-        step(std::true_type{}, b, d1, h1, d0, h0);
-        if (b + 1 < nb) step(std::true_type{}, b + 1, d0, h0, d1, h1);
+        gemm_mfma<MT, NMT, 1>(st + C::AB, w, lane, d, h);
+        gemm_fold<MT, NMT>(tl, lane, d, h, acc);
     }
-    if constexpr (!AHEAD) lds_barrier();
-    const int last = slot == 0 ? 2 : slot - 1;  // the slot of nb - 1
-    if (nb & 1)
-        gemm_fold<NMT>(tails + last * GM_TB, lane, d0, h0, acc);
-    else
-        gemm_fold<NMT>(tails + last * GM_TB, lane, d1, h1, acc);
 }
 
-__global__ __launch_bounds__(64 * GM_WAVES) void k_gemm_q4k(GemmArgs g) {
+// The loop on the 16-token tiles that hold `valid` tokens.
+template <bool HALVES, int MT, int NMT, int NT, class Issue, class Weights>
+SYN_DEV void gemm_tiles(int valid, int nb, uint8_t* smem, int lane, Issue&& issue, Weights&& weights,
+                        v4f (&acc)[MT][NT]) {
+    if constexpr (NMT < MT) {
+        if (valid > 16 * NMT) {
+            gemm_tiles<HALVES, MT, NMT + (MT > 4 ? 2 : 1), NT>(valid, nb, smem, lane, issue, weights, acc);
+            return;
+        }
+    }
+    gemm_loop<HALVES, MT, NMT, NT>(nb, smem, lane, issue, weights, acc);
+}
+
+template <bool HALVES, int MT, int NT>
+__global__ __launch_bounds__(64 * GM_WAVES, 2) void k_gemm_q4k(GemmArgs g) {
+    using C = GmCfg<MT>;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: slot choices in SGPRs
-    const int n0 = blockIdx.x * GM_ROWS, t0 = blockIdx.y * GM_TT;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: copy bases in SGPRs
+    const int c = lane & 15, p = lane >> 4;
+    const int per = g.xcd_tokens, id = (int)blockIdx.x >> 3;
+    const int nx = per ? id / per : (int)blockIdx.x;
+    const int ty = per ? ((int)blockIdx.x & 7) * per + id - nx * per : (int)blockIdx.y;
+    const int n0 = nx * gemm_rows(NT) + 16 * NT * wave, t0 = ty * C::TT;
     const int T = active_rows(g.active, 0, g.T);
     if (t0 >= T) return;  // uniform: a token tile past the step's active rows
-    const GemmSlots sl = gemm_slots(g, wave, lane, n0, t0);
-    const int live = sl.nw + GM_ASLOT / GM_WAVES + sl.nt;  // loads per stage of this wavefront
-    v4f acc[GM_MT][GM_NT];
+    const GemmSlots<MT> sl = gemm_slots<MT>(g.tpad, wave, lane, t0);
+    uint32_t off[NT], qoff[NT];
 #pragma unroll
-    for (int mt = 0; mt < GM_MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < GM_NT; ++nt) acc[mt][nt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-
-    auto issue = [&](int b, uint8_t* stage, uint8_t* tail) { gemm_issue(g, sl, wave, lane, b, t0, stage, tail); };
-    // the 16-token tiles holding active rows (a last tile of fewer rows computes only those)
-    switch ((T - t0 < GM_TT ? T - t0 + 15 : GM_TT) / 16) {
-        case 1: gemm_loop<1, true>(g.nb, live, smem, wave, lane, issue, acc); break;
-        case 2: gemm_loop<2, true>(g.nb, live, smem, wave, lane, issue, acc); break;
-        case 3: gemm_loop<3, true>(g.nb, live, smem, wave, lane, issue, acc); break;
-        default: gemm_loop<GM_MT, true>(g.nb, live, smem, wave, lane, issue, acc); break;
+    for (int nt = 0; nt < NT; ++nt) {
+        const int n = n0 + 16 * nt + c;
+        off[nt] = gemm_row_offset(g.layout, (uint32_t)(n < g.N ? n : g.N - 1), g.rb);
+        qoff[nt] = off[nt] + gemm_chunk_step(g.layout) * (uint32_t)(1 + 2 * p);
     }
+    v4f acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int c = lane & 15, p = lane >> 4;
+    auto issue = [&](auto half, int b, uint8_t* stage, uint8_t* tail) {
+        gemm_issue<MT, decltype(half)::value>(sl, g.codes + ((size_t)b * g.tpad + t0) * 512,
+                                              g.tail + (size_t)b * g.tpad * GM_TAIL_ROW, wave, lane, stage, tail);
+    };
+    // super-block b of row 0: in X8 block b sits in run b / 8 at position b % 8
+    auto weights = [&](int b) {
+        return gemm_weights(g.layout == LAYOUT_X8 ? g.W + 1152 * (size_t)(b >> 3) + 16 * (size_t)(b & 7)
+                                                  : g.W + 144 * (size_t)b,
+                            off, qoff, gemm_chunk_step(g.layout));
+    };
+    gemm_tiles<HALVES, MT, (MT > 4 ? 2 : 1), NT>(T - t0, g.nb, smem, lane, issue, weights, acc);
+
 #pragma unroll
-    for (int mt = 0; mt < GM_MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < GM_NT; ++nt) {
-            const int n = n0 + 16 * GM_NT * wave + 16 * nt + c;
+        for (int nt = 0; nt < NT; ++nt) {
+            const int n = n0 + 16 * nt + c;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int t = t0 + 16 * mt + 4 * p + i;
@@ -471,6 +527,42 @@ __global__ __launch_bounds__(64 * GM_WAVES) void k_gemm_q4k(GemmArgs g) {
 bool gemm_q4k_supported(int n_out, int k) {
     return k >= 256 && k % 256 == 0 && n_out > 0 &&
            (uint64_t)n_out * (uint64_t)(k / 256) * 144u < (1ull << 32);
+}
+
+// The wavefront tile.  A large one makes each weight operand once for more tokens and reads each token
+// once for more rows, a small one gives the SIMDs wavefronts: one alone issues a vector operation
+// every five cycles, two every two and a half.  Microseconds measured for 32 tokens x 16 rows | 64 x
+// 16 | 64 x 32 (whole super-blocks, halves) | 128 x 32, X8:
+//   4096 x 4096 at 64 rows (512 wavefronts of 32 x 16)   21 | 27 | 45, 44 | 48
+//   4096 x 4096 at 200 (1792)                            34 | 35 | 50, 49 | 75
+//   4096 x 4096 at 333 (2816; 1536 of 64 x 16)           53 | 47 | 54, 52 | 78
+//   14336 x 4096 at 200 (3584 of 64 x 16)               104 | 85 | 70, 80 | 82
+//   14336 x 4096 at 333 (336 workgroups of 128 x 128)   154 | 127 | 112, 110 | 97
+//   14336 x 4096 at 1024 (896)                          424 | 314 | 246, 255 | 215
+// X8 reaches the 128-token form first: a 16-byte chunk of a block shares its 128-byte line with seven
+// other blocks' chunks, so a workgroup draws eight times its weight bytes through its L1, and twice
+// the tokens halve that (GGUF at 512 rows, 448 workgroups: 113 against 119 with 64 x 32; at 333: 90 against 89).  64 x 32 with whole super-blocks holds two workgroups a CU, halves three: the former
+// while two hold them all.
+constexpr int64_t GM_SMALL_WAVES = 2048, GM_MID_WAVES = 3072, GM_WIDE_X8 = 320, GM_WIDE = 448;
+
+template <bool HALVES, int MT, int NT>
+static void launch_gemm_tiles(GemmArgs g, hipStream_t stream) {
+    using C = GmCfg<MT>;
+    // once per process, thread-safe (a function-local static); a refusal shows as the launch's error
+    static const hipError_t attr =
+        hipFuncSetAttribute((const void*)k_gemm_q4k<HALVES, MT, NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            C::template LDS<HALVES>);
+    (void)attr;
+    const unsigned nx = (unsigned)((g.N + gemm_rows(NT) - 1) / gemm_rows(NT)), ny = (unsigned)((g.T + C::TT - 1) / C::TT);
+    // Workgroups go to the 8 XCDs in turn.  Row tile by row tile, an XCD's L2 sees an eighth of the
+    // weights and all tokens; where the tokens are the larger operand (512 bytes a super-block
+    // against 144) and give every XCD as many tiles, an eighth of the tokens and all weights (GGUF 2048
+    // x 8192 at 2048 rows 145 against 155 us; X8, whose lines are read eight times, 4096 x 14336 451
+    // against 400).
+    g.xcd_tokens = g.layout != LAYOUT_X8 && ny % 8 == 0 && nx < (1u << 23) / ny &&
+                           (int64_t)g.T * 512 > (int64_t)g.N * 144 ? (int)(ny / 8) : 0;
+    const dim3 grid(g.xcd_tokens ? nx * ny : nx, g.xcd_tokens ? 1u : ny);
+    hipLaunchKernelGGL((k_gemm_q4k<HALVES, MT, NT>), grid, dim3(64 * GM_WAVES), C::template LDS<HALVES>, stream, g);
 }
 
 void launch_gemm_q4k(int layout, const uint8_t* W, int n_out, int k, GemmAct a, int T, float* y,
@@ -487,12 +579,17 @@ void launch_gemm_q4k(int layout, const uint8_t* W, int n_out, int k, GemmAct a, 
     g.nb = k / 256;
     g.tpad = a.tpad;
     g.rb = (uint32_t)(k / 256) * 144u;
-    // once per process, thread-safe (a function-local static); a refusal shows as the launch's error
-    static const hipError_t attr =
-        hipFuncSetAttribute((const void*)k_gemm_q4k, hipFuncAttributeMaxDynamicSharedMemorySize, GM_LOOP_LDS);
-    (void)attr;
-    const dim3 grid((unsigned)((n_out + GM_ROWS - 1) / GM_ROWS), (unsigned)(a.tpad / GM_TT));
-    hipLaunchKernelGGL(k_gemm_q4k, grid, dim3(64 * GM_WAVES), GM_LOOP_LDS, stream, g);
+    const int64_t n = n_out, t = T;
+    if ((n + 15) / 16 * ((t + 31) / 32) <= GM_SMALL_WAVES)
+        launch_gemm_tiles<false, 2, 1>(g, stream);
+    else if ((n + 15) / 16 * ((t + 63) / 64) <= (layout == LAYOUT_X8 ? GM_MID_WAVES : GM_MID_WAVES + 512))
+        launch_gemm_tiles<true, 4, 1>(g, stream);
+    else if ((n + 127) / 128 * ((t + 127) / 128) >= (layout == LAYOUT_X8 ? GM_WIDE_X8 : GM_WIDE))
+        launch_gemm_tiles<true, 8, 2>(g, stream);
+    else if ((n + 127) / 128 * ((t + 63) / 64) <= 512)
+        launch_gemm_tiles<false, 4, 2>(g, stream);
+    else
+        launch_gemm_tiles<true, 4, 2>(g, stream);
 }
 
 // ============================================================================================
@@ -506,11 +603,11 @@ void launch_gemm_q4k(int layout, const uint8_t* W, int n_out, int k, GemmAct a, 
 // (moe.rs:479-492), which depends on the row alone, so:
 //   gate/up: the tokens' rows are quantized to Q8_K once, in the GEMM layout, and each stage
 //     gathers position p's row from its entry's token (slots[i] / top_k); a workgroup takes
-//     (tile, 128 weight rows); its 256-row weight tile is those 128 rows of the tile's gate
-//     matrix followed by the same 128 rows of its up matrix, so wavefronts 0-3 hold g and
-//     wavefronts 4-7 hold u of the same outputs, and h = silu(g) * u per entry
+//     (tile, 64 weight rows); its 128-row weight tile is those 64 rows of the tile's gate
+//     matrix followed by the same 64 rows of its up matrix, so wavefronts 0-1 hold g and
+//     wavefronts 2-3 hold u of the same outputs, and h = silu(g) * u per entry
 //     (moe.rs:529-551);
-//   down: the entries' h rows quantized at their padded positions; (tile, 256 rows) of the
+//   down: the entries' h rows quantized at their padded positions; (tile, 128 rows) of the
 //     expert's down matrix; each output goes to its entry's slot (moe.rs:500-515).
 // Every product is the Gemv value (the same exact sums and term fold as the dense GEMM).
 
@@ -594,9 +691,12 @@ struct MoeGemmArgs {
                         // entry's token slots[i] / top_k
 };
 
-// MODE 0 (gate/up, 128 weight rows of each per workgroup) or 1 (down, 256 rows).
+constexpr int GM_MT = 4;  // 16-entry tiles of an entry tile
+constexpr int GM_NT = 2, GM_ROWS = gemm_rows(GM_NT);
+
+// MODE 0 (gate/up, 64 weight rows of each per workgroup) or 1 (down, 128 rows).
 template <int MODE>
-__global__ __launch_bounds__(64 * GM_WAVES) void k_moe_gemm(MoeGemmArgs g) {
+__global__ __launch_bounds__(64 * GM_WAVES, 3) void k_moe_gemm(MoeGemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     if (g.err[0]) return;
     const int tile = (int)blockIdx.x / g.row_tiles, rt = (int)blockIdx.x - tile * g.row_tiles;
@@ -609,84 +709,60 @@ __global__ __launch_bounds__(64 * GM_WAVES) void k_moe_gemm(MoeGemmArgs g) {
     const uint32_t left = g.offsets[e + 1] - i0;
     const int nvalid = left < 64u ? (int)left : 64;
     constexpr int ROWS = MODE == 0 ? GM_ROWS / 2 : GM_ROWS;  // rows of each matrix
-    const uint8_t* b0 = g.W0 + (uint64_t)e * g.ebytes + (uint64_t)rt * ROWS * g.rb;
-    const uint8_t* b1 = MODE == 0 ? g.W1 + (uint64_t)e * g.ebytes + (uint64_t)rt * ROWS * g.rb : b0;
-    // the weight tile's 256 rows: MODE 0 rows 0-127 of b0 then rows 0-127 of b1 (slots
-    // 0..GM_WSLOT/2-1 hold exactly the first 128 rows: 128 * 9 chunks = 18 slots of 64)
-    GemmArgs ga{};
-    ga.layout = g.layout;
-    ga.N = GM_ROWS;
-    ga.rb = g.rb;
-    ga.codes = g.act.codes;
-    ga.tail = g.act.tail;
-    ga.tpad = g.act.tpad;
-    ga.nb = g.nb;
-    GemmSlots sl = gemm_slots(ga, wave, lane, 0, t0);
-    static_assert(GM_ROWS / 2 * 9 % 64 == 0, "gate and up halves on whole slots");
-    constexpr int HALF_SLOTS = GM_ROWS / 2 * 9 / 64;
-    bool upper[GM_WPW];
+    using C = GmCfg<GM_MT>;
+    const int c = lane & 15, p = lane >> 4;
+    // MODE 0: wavefronts 0-1 take the gate matrix's rows, 2-3 the same rows of up
+    const bool upper = MODE == 0 && wave >= GM_WAVES / 2;
+    const uint8_t* wm = (upper ? g.W1 : g.W0) + (uint64_t)e * g.ebytes + (uint64_t)rt * ROWS * g.rb;
+    uint32_t off[GM_NT], qoff[GM_NT];
 #pragma unroll
-    for (int u = 0; u < GM_WPW; ++u) {
-        upper[u] = MODE == 0 && wave + GM_WAVES * u >= HALF_SLOTS;
-        if (upper[u]) sl.woff[u] -= (uint32_t)(GM_ROWS / 2) * g.rb;
+    for (int nt = 0; nt < GM_NT; ++nt) {
+        off[nt] = gemm_row_offset(g.layout, (uint32_t)(16 * GM_NT * (wave - (upper ? GM_WAVES / 2 : 0)) + 16 * nt + c), g.rb);
+        qoff[nt] = off[nt] + 16u * (uint32_t)(1 + 2 * p);
     }
-    // MODE 0 gathers each position's token row from the tokens' quantized rows: code slot u of
-    // this lane is 16-byte chunk q of position pa, which holds chunk q ^ (pa & 15) (the stage's
-    // bank skew) and sits in the token's row at chunk (q ^ (pa & 15)) ^ (tok & 15) (the row's
-    // own skew); tail: wavefronts 0-1 the s2 halves, 2 the scales, 3 the code sums, one position
-    // a lane (padding positions read token 0; their outputs are dropped)
+    // super-block b of the tile's rows: 144 b on in GGUF order, 64 rows' blocks on in TILE64
+    const size_t bstep = g.layout == LAYOUT_TILE64 ? (size_t)TILE64_ROWS * 144 : 144;
+    auto weights = [&](int b) { return gemm_weights(wm + bstep * (size_t)b, off, qoff, 16u); };
+    // MODE 0 gathers each position's token row from the tokens' quantized rows: a token's chunks are
+    // skewed by its own number, the stage's lines by the position's.  Tail: wavefronts 0-1 the s2
+    // halves, 2 the scales, 3 the code sums, one position a lane (padding positions read token 0;
+    // their outputs are dropped)
+    GemmSlots<GM_MT> sl = gemm_slots<GM_MT>(g.act.tpad, wave, lane, t0);
+    static_assert(C::TT == 64 && C::TPW == 1, "one tail part a wavefront");
     const uint32_t tp = (uint32_t)g.act.tpad;
     auto token_of = [&](int pa) -> uint32_t {
         return pa < nvalid ? g.slots[i0 + (uint32_t)pa] / (uint32_t)g.top_k : 0u;
     };
-    uint32_t aoff[GM_ASLOT / GM_WAVES];
-    uint32_t toff = 0;
+    uint32_t aoff[C::APW];
     if constexpr (MODE == 0) {
 #pragma unroll
-        for (int u = 0; u < GM_ASLOT / GM_WAVES; ++u) {
-            const int pa = 2 * (wave + GM_WAVES * u) + (lane >> 5), q = lane & 31;
-            const uint32_t tok = token_of(pa);
-            aoff[u] = tok * 512u + 16u * (uint32_t)((q ^ (pa & 15)) ^ (int)(tok & 15u));
+        for (int i = 0; i < C::APW; ++i) {
+            const int u = wave + GM_WAVES * i;
+            const uint32_t tok = token_of(4 * u + (lane >> 4));
+            aoff[i] = tok * 512u + 16u * gemm_achunk(u, lane, tok);
         }
-        if (wave < 2) {
-            toff = token_of((64 * wave + lane) >> 1) * 32u + 16u * (uint32_t)(lane & 1);
-        } else if (wave < 4) {
-            toff = tp * (wave == 2 ? 32u : 36u) + token_of(lane) * 4u;
-        }
+        sl.toff[0] = wave < 2 ? token_of((64 * wave + lane) >> 1) * 32u + 16u * (uint32_t)(lane & 1)
+                              : tp * (wave == 2 ? 32u : 36u) + token_of(lane) * 4u;
     }
-    // super-block b of the tile's rows: 144 b on in GGUF order, 64 rows' blocks on in TILE64
-    const size_t bstep = g.layout == LAYOUT_TILE64 ? (size_t)TILE64_ROWS * 144 : 144;
-    auto issue = [&](int b, uint8_t* stage, uint8_t* tail) {
-        const uint8_t* w0 = b0 + bstep * (size_t)b;
-        const uint8_t* w1 = b1 + bstep * (size_t)b;
-        const uint32_t st = lds_addr(stage);
-#pragma unroll
-        for (int u = 0; u < GM_WPW; ++u)
-            if (u < sl.nw) lds_dma16(sl.woff[u], upper[u] ? w1 : w0, st + 1024u * (uint32_t)(wave + GM_WAVES * u));
-        if constexpr (MODE == 0) {
-            // super-block bases in 64 bits (2 * hidden * tp bytes of codes may pass 2^32);
-            // the offsets within one super-block's rows stay below 2^25
-            const uint8_t* ab = g.act.codes + (size_t)b * tp * 512u;
-            const uint8_t* tb = g.act.tail + (size_t)b * tp * (uint32_t)GM_TAIL_ROW;
-#pragma unroll
-            for (int u = 0; u < GM_ASLOT / GM_WAVES; ++u) {
-                const int gs = wave + GM_WAVES * u;
-                lds_dma16(aoff[u], ab, st + (uint32_t)GM_WB + 1024u * (uint32_t)gs);
-            }
-            const uint32_t tl = lds_addr(tail);
-            if (wave < 2)
-                lds_dma16(toff, tb, tl + 1024u * (uint32_t)wave);
-            else if (wave < 4)
-                lds_dma4(toff, tb, tl + (wave == 2 ? 2048u : 2304u));
+    auto issue = [&](auto half, int b, uint8_t* stage, uint8_t* tail) {
+        constexpr int H = decltype(half)::value;
+        // super-block bases in 64 bits (2 * hidden * tp bytes of codes may pass 2^32); the offsets
+        // within one super-block's rows stay below 2^25
+        const uint8_t* ab = g.act.codes + ((size_t)b * tp + (MODE == 0 ? 0 : t0)) * 512u;
+        const uint8_t* tb = g.act.tail + (size_t)b * tp * (uint32_t)GM_TAIL_ROW;
+        if constexpr (MODE == 1) {
+            gemm_issue<GM_MT, H>(sl, ab, tb, wave, lane, stage, tail);
         } else {
-            const uint8_t* ab = g.act.codes + ((size_t)b * g.act.tpad + t0) * 512;
-            const uint8_t* tb = g.act.tail + (size_t)b * g.act.tpad * GM_TAIL_ROW;
+            const uint32_t tl = lds_addr(tail);
 #pragma unroll
-            for (int u = 0; u < GM_ASLOT / GM_WAVES; ++u) {
-                const int gs = wave + GM_WAVES * u;
-                lds_dma16(16u * (uint32_t)lane, ab + 1024 * gs, st + (uint32_t)GM_WB + 1024u * (uint32_t)gs);
+            for (int i = 0; i < C::APW; ++i)
+                lds_dma16(aoff[i] ^ (64u * H), ab, lds_addr(stage) + 1024u * (uint32_t)(wave + GM_WAVES * i));
+            if constexpr (H == 1) {
+                if (wave < 2)
+                    lds_dma16(sl.toff[0], tb, tl + 1024u * (uint32_t)wave);
+                else
+                    lds_dma4(sl.toff[0], tb, tl + (wave == 2 ? 2048u : 2304u));
             }
-            if (sl.ton) lds_dma16(sl.toff, tb, lds_addr(tail) + 1024u * (uint32_t)wave);
         }
     };
     v4f acc[GM_MT][GM_NT];
@@ -696,16 +772,11 @@ __global__ __launch_bounds__(64 * GM_WAVES) void k_moe_gemm(MoeGemmArgs g) {
         for (int nt = 0; nt < GM_NT; ++nt) acc[mt][nt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     // the 16-token tiles holding entries (the padding of an expert's last tile is not computed;
     // its outputs are dropped)
-    switch ((nvalid + 15) / 16) {
-        case 1: gemm_loop<1, false>(g.nb, 0, smem, wave, lane, issue, acc); break;
-        case 2: gemm_loop<2, false>(g.nb, 0, smem, wave, lane, issue, acc); break;
-        case 3: gemm_loop<3, false>(g.nb, 0, smem, wave, lane, issue, acc); break;
-        default: gemm_loop<GM_MT, false>(g.nb, 0, smem, wave, lane, issue, acc); break;
-    }
-    const int c = lane & 15, p = lane >> 4;
+    gemm_tiles<true, GM_MT, 1, GM_NT>(nvalid, g.nb, smem, lane, issue, weights, acc);
     if constexpr (MODE == 0) {
-        // u (wavefronts 4-7) through LDS to the wavefronts holding g of the same outputs
-        float* ux = reinterpret_cast<float*>(smem);  // [64 tokens][128 rows]
+        // u (the upper wavefronts) through LDS to the wavefronts holding g of the same outputs
+        float* ux = reinterpret_cast<float*>(smem);  // [64 tokens][64 rows]
+        lds_barrier();                               // the last stage is read out
         if (wave >= GM_WAVES / 2) {
 #pragma unroll
             for (int mt = 0; mt < GM_MT; ++mt)
@@ -746,7 +817,7 @@ __global__ __launch_bounds__(64 * GM_WAVES) void k_moe_gemm(MoeGemmArgs g) {
 void launch_moe_gemm(int mode, const uint8_t* w0, const uint8_t* w1, int n_experts, int rows, int k,
                      GemmAct act, int max_tiles, const uint32_t* offsets, MoeTiles mt, const uint32_t* err,
                      const uint32_t* slots, float* out, hipStream_t stream, int top_k, int layout) {
-    static_assert(GM_ROWS % (2 * TILE64_ROWS) == 0, "row tiles of whole TILE64 runs");
+    static_assert(GM_ROWS == 2 * TILE64_ROWS, "row tiles of whole TILE64 runs");
     MoeGemmArgs g;
     g.top_k = top_k;
     g.layout = layout == LAYOUT_TILE64 ? (int)LAYOUT_TILE64 : (int)LAYOUT_SOURCE;
@@ -766,18 +837,18 @@ void launch_moe_gemm(int mode, const uint8_t* w0, const uint8_t* w1, int n_exper
     const dim3 grid((unsigned)(max_tiles * g.row_tiles));
     if (mode == 0) {
         static const hipError_t ok0 = hipFuncSetAttribute((const void*)k_moe_gemm<0>,
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, GM_LOOP_LDS);
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, GmCfg<GM_MT>::LDS<true>);
         (void)ok0;  // a refusal shows as the launch's error
-        hipLaunchKernelGGL(k_moe_gemm<0>, grid, dim3(64 * GM_WAVES), GM_LOOP_LDS, stream, g);
+        hipLaunchKernelGGL(k_moe_gemm<0>, grid, dim3(64 * GM_WAVES), GmCfg<GM_MT>::LDS<true>, stream, g);
     } else {
         static const hipError_t ok1 = hipFuncSetAttribute((const void*)k_moe_gemm<1>,
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, GM_LOOP_LDS);
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, GmCfg<GM_MT>::LDS<true>);
         (void)ok1;
-        hipLaunchKernelGGL(k_moe_gemm<1>, grid, dim3(64 * GM_WAVES), GM_LOOP_LDS, stream, g);
+        hipLaunchKernelGGL(k_moe_gemm<1>, grid, dim3(64 * GM_WAVES), GmCfg<GM_MT>::LDS<true>, stream, g);
     }
 }
 
-// Row tiles: gate/up 128 rows, down 256.
+// Row tiles: gate/up 64 rows, down 128.
 bool moe_gemm_supported(int hidden, int inter) { return hidden % GM_ROWS == 0 && inter % (GM_ROWS / 2) == 0; }
 
 }  // namespace syn

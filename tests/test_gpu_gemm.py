@@ -55,6 +55,24 @@ def test_gemm_equals_oracle(S, rows, n_out, k):
     assert_same(y2, want, "split gemm")
 
 
+@pytest.mark.parametrize("rows,n_out,k,x8", [
+    (33, 70, 512, False), (95, 1001, 256, False), (64, 129, 2048, True),   # 32 tokens x 16 rows a wavefront
+    (1100, 1039, 256, False), (577, 2049, 2048, True),                      # 64 x 16
+    (1000, 3201, 256, False), (961, 3195, 2048, True),                      # 64 x 32, whole super-blocks
+    (2200, 2047, 512, False), (2113, 1985, 2048, True),                     # 64 x 32, halves
+    (2689, 2999, 512, False), (2600, 2500, 2048, True),                     # 128 x 32, a tile past the padding
+    (1024, 700, 256, False), (2560, 2700, 256, False), (3072, 2690, 768, False)])  # an XCD's share of the tokens
+def test_gemm_wavefront_tiles(S, rows, n_out, k, x8):
+    """Each wavefront tile the product is dispatched to, at ragged sizes, over both weight orders."""
+    rs = np.random.default_rng(rows + n_out + k)
+    w = random_q4k(rs, n_out, k)
+    x = o.normal(0x6E21 + rows + k, 1.0, rows * k).reshape(rows, k)
+    W = S.Weights(S.WeightType.Q4K, dev(w), n_out, k)
+    announce(f"gemm tiles rows={rows} n_out={n_out} k={k} x8={x8}")
+    got = host(S.gemv(S.repack(W) if x8 else W, dev(x.astype(np.float32)), rows))
+    assert_same(got, o.gemv(o.Q4_K, w, n_out, k, x, rows, threads=16), "tiles")
+
+
 def test_gemm_extreme_magnitudes(S):
     """Scales 63 and codes 15 against codes +-127 of one sign: the largest sums the exact F16
     accumulation has to carry (256 * 127 * 512 < 2^24), and the smallest (codes 0)."""
