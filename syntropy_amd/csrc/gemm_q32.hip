@@ -20,6 +20,11 @@
 // Q4_0: the int8 operand holds 16 (n - 8) (a nibble in the high half of its byte, its top bit
 // flipped), and the scale is dw / 16: the same bound on s, the same exactness.
 //
+// Per 32 x 32 tile and block that is about 96 cycles of matrix products and 80 of vector operations, and
+// the two add up on this chip (two wavefronts a SIMD: a loop of both alone takes 184).  Measured, with
+// the operands' reads: about 250; 4096 x 14336 Q8_0 SPLIT at 512 rows 128 us against 155 for the
+// four-operation form (gemv_split.hip), GGUF Q4_0 6144 x 4096 at 200 rows 59 us against 841.
+//
 // A wavefront takes 32 rows x 32 TT tokens of one matrix, a workgroup RG x TG of them (gate and up: of
 // both matrices; the wavefronts that hold up hand it through LDS to those that hold gate).
 // Four blocks of every operand a stage are copied into LDS by global_load_lds one stage ahead.
@@ -205,9 +210,9 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
         }
 #pragma unroll
         for (int i = 0; i < C::DPW; ++i) doff[i] = token((64 * nth(i, C::DJ) + lane) % C::TOK) * (uint32_t)nb;
-        auto issue = [&](int sn) {
+        auto issue = [&](int sn, int slot) __attribute__((always_inline)) {
             const int s = sn < nst ? sn : nst - 1;  // a stage past the row repeats the last, so that the counts stay
-            const uint32_t st = ring + (uint32_t)(C::STAGE * (sn % C::NS));
+            const uint32_t st = ring + (uint32_t)(C::STAGE * slot);
 #pragma unroll
             for (int i = 0; i < C::WPW; ++i) {
                 const int u = nth(i, C::WJ);
@@ -287,7 +292,7 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
             }
             return x;
         };
-        auto make_row = [&](const RowRaw& x, int s, int j) __attribute__((always_inline)) {
+        auto make_row = [&](auto whole, const RowRaw& x, int s, int j) __attribute__((always_inline)) {
             uint32_t w[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -296,15 +301,15 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
                     w[i] = __builtin_amdgcn_bitop3_b32(w[i] << (h ? 0u : 4u), 0xF0F0F0F0u, 0x80808080u, 0x6A);  // (a & b) ^ c
             }
             return Row{v4i_q{(int)w[0], (int)w[1], (int)w[2], (int)w[3]},
-                       f16_to_f32(x.d16 & (G32_S * s + j < nb ? 0xFFFFu : 0u)) * unit};
+                       f16_to_f32(decltype(whole)::value || G32_S * s + j < nb ? x.d16 : 0u) * unit};
         };
         auto read_tok = [&](const uint8_t* st, int j, int t) __attribute__((always_inline)) {
             const int lt = 32 * (TT * tg + t) + c;
             return Tok{*reinterpret_cast<const v4i_q*>(st + C::A_OFF + lt * 128 + 16 * ((2 * j + h) ^ (lt & 7))),
                        *reinterpret_cast<const uint32_t*>(st + C::DX_OFF + 4 * (j * C::TOK + lt))};
         };
-        auto scale_of = [&](const Tok& x, int s, int j) __attribute__((always_inline)) {
-            return u2f(x.dx & (G32_S * s + j < nb ? 0xFFFFFFFFu : 0u));
+        auto scale_of = [&](auto whole, const Tok& x, int s, int j) __attribute__((always_inline)) {
+            return u2f(decltype(whole)::value || G32_S * s + j < nb ? x.dx : 0u);
         };
         // A tile's products (M + s and the two scale products) and its fold, a tile apart: the matrix
         // cores work on one tile while the vector ALU folds the one before.  The compiler's own order
@@ -318,18 +323,20 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
             for (int i = lo; i < hi; ++i) a[i] = a[i] + __builtin_fmaf(pc[k][i], u2f((uint32_t)f[k][i]), pc[k][16 + i]);
         };
 #pragma unroll
-        for (int s = 0; s < C::NS - 1; ++s) issue(s);
-        auto arrive = [&](int s) __attribute__((always_inline)) {
+        for (int s = 0; s < C::NS - 1; ++s) issue(s, s);
+        auto arrive = [&](int s, int slot) __attribute__((always_inline)) {
             wait_vm<C::COPIES * (C::NS - 2)>();  // this wavefront's copies of stage s have landed
             lds_barrier();                       // everyone's have, and stage s - 1 is read out
-            issue(s + C::NS - 1);
+            issue(s + C::NS - 1, (slot + C::NS - 1) % C::NS);
         };
         // NT: the 32-token tiles of this wavefront that hold tokens
         auto loop = [&](auto tiles) __attribute__((always_inline)) {
             constexpr int NT = decltype(tiles)::value, UNITS = G32_S * NT;  // an even number
-            for (int s = 0; s < nst; ++s) {
-                arrive(s);
-                const uint8_t* st = lds + C::STAGE * (s % C::NS);
+            // whole: every block of the stage is the row's (no scale to clear); slot: a constant
+            // where one token tile leaves registers, so that the LDS offsets are the instructions' own
+            auto stage = [&](auto whole, int s, int slot) __attribute__((always_inline)) {
+                arrive(s, slot);
+                const uint8_t* st = lds + C::STAGE * slot;
                 RowRaw wr = read_row(st, s, 0);
                 Row w;
                 Tok x = read_tok(st, 0, 0);
@@ -337,8 +344,8 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
                 for (int u = 0; u < UNITS; ++u) {
                     const int j = u / NT, t = u % NT, k = u & 1;
                     v16f_q& prev = acc[(u + UNITS - 1) % NT];
-                    if (t == 0) w = make_row(wr, s, j);
-                    float dx = scale_of(x, s, j);
+                    if (t == 0) w = make_row(whole, wr, s, j);
+                    float dx = scale_of(whole, x, s, j);
                     asm volatile("" : "+v"(w.a), "+v"(prev));
                     f[k] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w.a, x.b, bias, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
@@ -355,11 +362,24 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
                     asm volatile("" : "+v"(prev));
                     __builtin_amdgcn_sched_barrier(0);
                 }
+            };
+            if constexpr (TT == 1) {
+                const int nw = nb / G32_S;  // whole stages
+                for (int s = 0; s < nw; s += C::NS) {
+#pragma unroll
+                    for (int i = 0; i < C::NS; ++i) {
+                        if (s + i >= nw) break;  // uniform
+                        stage(std::true_type{}, s + i, i);
+                    }
+                }
+                if (nw < nst) stage(std::false_type{}, nw, nw % C::NS);
+            } else {  // (two token tiles leave no registers for it)
+                for (int s = 0; s < nst; ++s) stage(std::false_type{}, s, s % C::NS);
             }
             fold(acc[NT - 1], 1, 0, 16);
         };
         if (!busy)
-            for (int s = 0; s < nst; ++s) arrive(s);
+            for (int s = 0; s < nst; ++s) arrive(s, s % C::NS);
         else if (TT == 1 || valid - 32 * TT * tg > 32)
             loop(std::integral_constant<int, TT>{});
         else

@@ -1075,8 +1075,9 @@ void launch_gemm_q8_split(int ty, const uint8_t* W, int n_out, int k, const uint
         launch_staged_fmt<T_Q8_0>(W, n_out, k, xq, xd, T, y, stream, active);
         return;
     }
-    // other shapes: the register-staged kernel; up to 64 tokens: 16-token tiles; beyond, 32-token tiles (a token tile per wavefront, up to
-    // four wavefronts on the same 16 rows)
+    // a matrix or activation rows past gemm_q32.hip's 32-bit offsets: the register-staged kernel; up to 64
+    // tokens: 16-token tiles; beyond, 32-token tiles (a token tile per wavefront, up to four wavefronts on
+    // the same 16 rows)
     const int TT = T <= 64 ? 1 : 2;
     const int tiles = (T + 16 * TT - 1) / (16 * TT);
     const int wpw = tiles < 4 ? tiles : 4;

@@ -6,7 +6,10 @@
 // block the exact I32 sum s and the term (dw * dx) * s, the terms added in ascending block order
 // from +0.0 (gemv.rs:539-547, portable.rs:114-190).
 //
-// Mapping.  A workgroup takes one expert and 64 output rows (four wavefronts of 16 rows; four
+// The quantizer of the entries' rows, and the products where a matrix passes the 32-bit offsets of
+// gemm_q32.hip, which takes every other layer.
+//
+// Mapping of the products.  A workgroup takes one expert and 64 output rows (four wavefronts of 16 rows; four
 // lanes per row take the row's blocks in turn, block b to lane b mod 4, and hand the running
 // sum on with a DPP rotation, so the fold stays in block order).  It walks the expert's entries
 // eight at a time; each pass streams the rows' weights once, 16 blocks per stage through a
