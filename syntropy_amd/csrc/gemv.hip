@@ -271,25 +271,38 @@ void launch_gemv_q(int ty, const uint8_t* W, int n_out, int k, const uint8_t* ws
 // GateUpAct{Silu}: y[r][i] = silu(y2[r][i]) * y2[r][n + i], y2 the Gemv of the stacked
 // [gate; up] weight (crates/kernels/src/reference/linear.rs:75-112 with the quantized dots of
 // the MoE FFN, crates/kernels-cpu/src/moe.rs:529-551: software-exp silu, the product rounded
-// once).  Four outputs per thread.
-__global__ __launch_bounds__(256) void k_silu_mul(const float* __restrict__ y2, int rows, int n,
-                                                  float* __restrict__ y, const uint32_t* __restrict__ active) {
+// once).  A thread takes four neighbouring columns of a row (16-byte accesses where the rows' starts
+// allow them), a workgroup of one wavefront 256: the rows and columns come from the grid, with no
+// division a value.  333 x 5632 8.4 -> 5.0 us, the whole GateUpAct at 6 x 14336 24.6 -> 23.6.
+constexpr unsigned SILU_MAX_Y = 32768;
+
+template <bool VEC>
+__global__ __launch_bounds__(64) void k_silu_mul(const float* __restrict__ y2, int rows, int n,
+                                                 float* __restrict__ y, const uint32_t* __restrict__ active) {
     rows = active_rows(active, 0, rows);
-    const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int64_t i = i0 + q;
-        if (i >= (int64_t)rows * n) return;
-        const int64_t r = i / n, c = i - r * n;
-        y[i] = ref_silu(y2[r * 2 * n + c]) * y2[r * 2 * n + n + c];
+    const int c = ((int)blockIdx.x * 64 + (int)threadIdx.x) * 4;
+    if (c >= n) return;
+    for (int r = (int)blockIdx.y; r < rows; r += (int)gridDim.y) {
+        const float* g = y2 + (int64_t)r * 2 * n + c;
+        float* o = y + (int64_t)r * n + c;
+        if constexpr (VEC) {
+            const float4 gv = *reinterpret_cast<const float4*>(g), uv = *reinterpret_cast<const float4*>(g + n);
+            *reinterpret_cast<float4*>(o) = make_float4(ref_silu(gv.x) * uv.x, ref_silu(gv.y) * uv.y,
+                                                        ref_silu(gv.z) * uv.z, ref_silu(gv.w) * uv.w);
+        } else {
+            const int left = n - c < 4 ? n - c : 4;
+            for (int q = 0; q < left; ++q) o[q] = ref_silu(g[q]) * g[n + q];
+        }
     }
 }
 
 void launch_silu_mul(const float* y2, int rows, int n, float* y, hipStream_t stream, const uint32_t* active) {
-    const int64_t total = (int64_t)rows * n;
-    if (total == 0) return;
-    hipLaunchKernelGGL(k_silu_mul, dim3((unsigned)((total + 1023) / 1024)), dim3(256), 0, stream, y2, rows, n, y,
-                       active);
+    if (rows == 0 || n == 0) return;
+    const dim3 grid(((unsigned)n + 255) / 256, (unsigned)rows < SILU_MAX_Y ? (unsigned)rows : SILU_MAX_Y);
+    if (n % 4 == 0 && (((uintptr_t)y2 | (uintptr_t)y) & 15) == 0)
+        hipLaunchKernelGGL(k_silu_mul<true>, grid, dim3(64), 0, stream, y2, rows, n, y, active);
+    else
+        hipLaunchKernelGGL(k_silu_mul<false>, grid, dim3(64), 0, stream, y2, rows, n, y, active);
 }
 
 }  // namespace syn
