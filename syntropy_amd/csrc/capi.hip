@@ -632,7 +632,7 @@ bool staged_faster(int32_t wtype, uint32_t n_out, uint32_t k_in, uint32_t rows) 
 }
 
 // Rows on the int8 matrix cores: where the LDS-staged GEMM takes the shape and is the faster
-// (above), else Q8_0 from 9 rows on the register-staged GEMM.
+// (above), else (rows that are not whole stages) from where gemm_q32.hip is the faster.
 bool split_gemm(int32_t wtype, uint32_t n_out, uint32_t k_in, uint32_t rows) {
     if (wtype != SYN_Q8_0 && wtype != SYN_Q4_0) return false;
     if (rows >= 2 && syn::gemm_q8_staged_fits((int)wtype, (int)n_out, (int)k_in, (int)rows))
