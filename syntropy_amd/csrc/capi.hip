@@ -878,6 +878,18 @@ int syn_gate_up_act_rows(uint32_t layout, int32_t wtype, const void* w, uint64_t
         syn::launch_gate_up_q4k_f32((const uint8_t*)w, (int)n_out, (int)k_in, x, y, (hipStream_t)stream, active);
         return check_launch(W);
     }
+    // many rows of Q4_K: one product whose wavefronts hold gate and up of the same outputs (what it does
+    // not take, a refused call among that, goes on below)
+    if ((layout == SYN_LAYOUT_SOURCE || (layout == SYN_LAYOUT_X8 && k_in % 2048 == 0)) &&
+        use_gemm(wtype, rows, 2 * n_out, k_in) && w && x && aligned(w, 16) && aligned(x, 16) &&
+        w_bytes >= 2ull * n_out * (k_in / 256) * 144 && syn::gemm_q4k_gate_up_fits((int)layout, (int)n_out, (int)rows)) {
+        const syn::GemmAct a = syn::gemm_act_at((uint8_t*)ws, (int64_t)gemm_tpad(rows), (int)k_in);
+        syn::launch_gemm_act(x, (int)rows, (int)k_in, a, (hipStream_t)stream, active);
+        if (int rc = check_launch(W)) return rc;
+        syn::launch_gemm_q4k_gate_up((int)layout, (const uint8_t*)w, (int)n_out, (int)k_in, a, (int)rows, y,
+                                     (hipStream_t)stream, active);
+        return check_launch(W);
+    }
     uint64_t g = 0;
     (void)syn_gemv_layout_workspace_bytes(layout, wtype, rows, k_in, &g);
     float* y2 = (float*)((uint8_t*)ws + syn::align_up(g, 256));

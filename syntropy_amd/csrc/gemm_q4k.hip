@@ -472,8 +472,11 @@ SYN_DEV void gemm_tiles(int valid, int nb, uint8_t* smem, int lane, Issue&& issu
     gemm_loop<HALVES, MT, NMT, NT>(nb, smem, lane, issue, weights, acc);
 }
 
-template <bool HALVES, int MT, int NT>
+// GU: W stacks N / 2 gate rows and as many up rows; a wavefront's two row tiles are 16 gate rows and
+// the same up rows, and y[t][N / 2] = silu(gate) * up (the product k_silu_mul makes of a written y).
+template <bool HALVES, int MT, int NT, bool GU>
 __global__ __launch_bounds__(64 * GM_WAVES, 2) void k_gemm_q4k(GemmArgs g) {
+    static_assert(!GU || NT == 2, "a gate tile and an up tile");
     using C = GmCfg<MT>;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const int lane = threadIdx.x & 63;
@@ -482,15 +485,16 @@ __global__ __launch_bounds__(64 * GM_WAVES, 2) void k_gemm_q4k(GemmArgs g) {
     const int per = g.xcd_tokens, id = (int)blockIdx.x >> 3;
     const int nx = per ? id / per : (int)blockIdx.x;
     const int ty = per ? ((int)blockIdx.x & 7) * per + id - nx * per : (int)blockIdx.y;
-    const int n0 = nx * gemm_rows(NT) + 16 * NT * wave, t0 = ty * C::TT;
+    const int cols = GU ? g.N / 2 : g.N;
+    const int n0 = GU ? nx * (gemm_rows(NT) / 2) + 16 * wave : nx * gemm_rows(NT) + 16 * NT * wave, t0 = ty * C::TT;
     const int T = active_rows(g.active, 0, g.T);
     if (t0 >= T) return;  // uniform: a token tile past the step's active rows
     const GemmSlots<MT> sl = gemm_slots<MT>(g.tpad, wave, lane, t0);
     uint32_t off[NT], qoff[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        const int n = n0 + 16 * nt + c;
-        off[nt] = gemm_row_offset(g.layout, (uint32_t)(n < g.N ? n : g.N - 1), g.rb);
+        const int n = n0 + (GU ? 0 : 16 * nt) + c;
+        off[nt] = gemm_row_offset(g.layout, (uint32_t)((n < cols ? n : cols - 1) + (GU ? nt * cols : 0)), g.rb);
         qoff[nt] = off[nt] + gemm_chunk_step(g.layout) * (uint32_t)(1 + 2 * p);
     }
     v4f acc[MT][NT];
@@ -514,12 +518,13 @@ __global__ __launch_bounds__(64 * GM_WAVES, 2) void k_gemm_q4k(GemmArgs g) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
+        for (int nt = 0; nt < (GU ? 1 : NT); ++nt) {
             const int n = n0 + 16 * nt + c;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int t = t0 + 16 * mt + 4 * p + i;
-                if (t < T && n < g.N) g.y[(int64_t)t * g.N + n] = acc[mt][nt][i];
+                if (t < T && n < cols)
+                    g.y[(int64_t)t * cols + n] = GU ? ref_silu(acc[mt][0][i]) * acc[mt][NT - 1][i] : acc[mt][nt][i];
             }
         }
 }
@@ -545,15 +550,16 @@ bool gemm_q4k_supported(int n_out, int k) {
 // while two hold them all.
 constexpr int64_t GM_SMALL_WAVES = 2048, GM_MID_WAVES = 3072, GM_WIDE_X8 = 320, GM_WIDE = 448;
 
-template <bool HALVES, int MT, int NT>
+template <bool HALVES, int MT, int NT, bool GU = false>
 static void launch_gemm_tiles(GemmArgs g, hipStream_t stream) {
     using C = GmCfg<MT>;
     // once per process, thread-safe (a function-local static); a refusal shows as the launch's error
     static const hipError_t attr =
-        hipFuncSetAttribute((const void*)k_gemm_q4k<HALVES, MT, NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipFuncSetAttribute((const void*)k_gemm_q4k<HALVES, MT, NT, GU>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             C::template LDS<HALVES>);
     (void)attr;
-    const unsigned nx = (unsigned)((g.N + gemm_rows(NT) - 1) / gemm_rows(NT)), ny = (unsigned)((g.T + C::TT - 1) / C::TT);
+    const int cols = GU ? g.N / 2 : g.N, wide = GU ? gemm_rows(NT) / 2 : gemm_rows(NT);
+    const unsigned nx = (unsigned)((cols + wide - 1) / wide), ny = (unsigned)((g.T + C::TT - 1) / C::TT);
     // Workgroups go to the 8 XCDs in turn.  Row tile by row tile, an XCD's L2 sees an eighth of the
     // weights and all tokens; where the tokens are the larger operand (512 bytes a super-block
     // against 144) and give every XCD as many tiles, an eighth of the tokens and all weights (GGUF 2048
@@ -562,11 +568,11 @@ static void launch_gemm_tiles(GemmArgs g, hipStream_t stream) {
     g.xcd_tokens = g.layout != LAYOUT_X8 && ny % 8 == 0 && nx < (1u << 23) / ny &&
                            (int64_t)g.T * 512 > (int64_t)g.N * 144 ? (int)(ny / 8) : 0;
     const dim3 grid(g.xcd_tokens ? nx * ny : nx, g.xcd_tokens ? 1u : ny);
-    hipLaunchKernelGGL((k_gemm_q4k<HALVES, MT, NT>), grid, dim3(64 * GM_WAVES), C::template LDS<HALVES>, stream, g);
+    hipLaunchKernelGGL((k_gemm_q4k<HALVES, MT, NT, GU>), grid, dim3(64 * GM_WAVES), C::template LDS<HALVES>, stream, g);
 }
 
-void launch_gemm_q4k(int layout, const uint8_t* W, int n_out, int k, GemmAct a, int T, float* y,
-                     hipStream_t stream, const uint32_t* active) {
+static GemmArgs gemm_args(int layout, const uint8_t* W, int n_out, int k, GemmAct a, int T, float* y,
+                          const uint32_t* active) {
     GemmArgs g{};
     g.active = active;
     g.W = W;
@@ -579,17 +585,47 @@ void launch_gemm_q4k(int layout, const uint8_t* W, int n_out, int k, GemmAct a, 
     g.nb = k / 256;
     g.tpad = a.tpad;
     g.rb = (uint32_t)(k / 256) * 144u;
+    return g;
+}
+
+static bool gemm_mid(int layout, int64_t n, int64_t t) {
+    return (n + 15) / 16 * ((t + 63) / 64) <= (layout == LAYOUT_X8 ? GM_MID_WAVES : GM_MID_WAVES + 512);
+}
+
+template <bool GU>
+static void launch_gemm_wide(const GemmArgs& g, hipStream_t stream) {
+    const int64_t n = g.N, t = g.T;
+    if ((n + 127) / 128 * ((t + 127) / 128) >= (g.layout == LAYOUT_X8 ? GM_WIDE_X8 : GM_WIDE))
+        launch_gemm_tiles<true, 8, 2, GU>(g, stream);
+    else if ((n + 127) / 128 * ((t + 63) / 64) <= 512)
+        launch_gemm_tiles<false, 4, 2, GU>(g, stream);
+    else
+        launch_gemm_tiles<true, 4, 2, GU>(g, stream);
+}
+
+void launch_gemm_q4k(int layout, const uint8_t* W, int n_out, int k, GemmAct a, int T, float* y,
+                     hipStream_t stream, const uint32_t* active) {
+    const GemmArgs g = gemm_args(layout, W, n_out, k, a, T, y, active);
     const int64_t n = n_out, t = T;
     if ((n + 15) / 16 * ((t + 31) / 32) <= GM_SMALL_WAVES)
         launch_gemm_tiles<false, 2, 1>(g, stream);
-    else if ((n + 15) / 16 * ((t + 63) / 64) <= (layout == LAYOUT_X8 ? GM_MID_WAVES : GM_MID_WAVES + 512))
+    else if (gemm_mid(layout, n, t))
         launch_gemm_tiles<true, 4, 1>(g, stream);
-    else if ((n + 127) / 128 * ((t + 127) / 128) >= (layout == LAYOUT_X8 ? GM_WIDE_X8 : GM_WIDE))
-        launch_gemm_tiles<true, 8, 2>(g, stream);
-    else if ((n + 127) / 128 * ((t + 63) / 64) <= 512)
-        launch_gemm_tiles<false, 4, 2>(g, stream);
     else
-        launch_gemm_tiles<true, 4, 2>(g, stream);
+        launch_gemm_wide<false>(g, stream);
+}
+
+// Where the product takes tiles of two 16-row tiles a wavefront: GateUpAct's gate and up then meet in
+// one (no [T][2 n] product written and read back: 5632 x 2048 at 333 rows 43.1 -> 38.8 us); below, the
+// smaller tiles and k_silu_mul.
+bool gemm_q4k_gate_up_fits(int layout, int n, int T) {
+    const int64_t n2 = 2 * (int64_t)n;
+    return (n2 + 15) / 16 * ((T + 31) / 32) > GM_SMALL_WAVES && !gemm_mid(layout, n2, T);
+}
+
+void launch_gemm_q4k_gate_up(int layout, const uint8_t* W, int n, int k, GemmAct a, int T, float* y,
+                             hipStream_t stream, const uint32_t* active) {
+    launch_gemm_wide<true>(gemm_args(layout, W, 2 * n, k, a, T, y, active), stream);
 }
 
 // ============================================================================================

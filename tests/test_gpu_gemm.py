@@ -73,6 +73,22 @@ def test_gemm_wavefront_tiles(S, rows, n_out, k, x8):
     assert_same(got, o.gemv(o.Q4_K, w, n_out, k, x, rows, threads=16), "tiles")
 
 
+@pytest.mark.parametrize("rows,n,k,x8", [
+    (1000, 1805, 256, False), (993, 1601, 2048, True),     # 64 x 32, whole super-blocks
+    (2200, 1025, 256, False), (2177, 1031, 2048, True),    # halves
+    (2600, 1499, 256, False), (2561, 1281, 2048, True),    # 128 x 32
+    (3072, 1345, 256, False)])                             # an XCD's share of the tokens
+def test_gate_up_in_one_product(S, rows, n, k, x8):
+    """GateUpAct where gate and up rows meet in a wavefront, at ragged sizes, over both weight orders."""
+    rs = np.random.default_rng(rows + n + k)
+    w = random_q4k(rs, 2 * n, k)
+    x = o.normal(0x6E31 + rows + k, 0.1, rows * k).reshape(rows, k)
+    W = S.Weights(S.WeightType.Q4K, dev(w), 2 * n, k)
+    announce(f"gate_up product rows={rows} n={n} k={k} x8={x8}")
+    got = host(S.gate_up_act(S.repack(W) if x8 else W, dev(x.astype(np.float32)), rows))
+    assert_same(got, o.gate_up_act(o.Q4_K, w, n, k, x, rows, threads=16), "gate_up")
+
+
 def test_gemm_extreme_magnitudes(S):
     """Scales 63 and codes 15 against codes +-127 of one sign: the largest sums the exact F16
     accumulation has to carry (256 * 127 * 512 < 2^24), and the smallest (codes 0)."""
