@@ -391,16 +391,29 @@ SYN_DEV uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(lds_ptr)
 // 16 bytes per active lane from sbase + voff to LDS address lds + 16 * lane, with no registers
 // held while the load flies.  Written as assembly so the compiler does not track it (it would
 // otherwise wait for every load into LDS in flight before each LDS read); the caller waits with
-// wait_vm.  The LDS address is an m0 operand, so the compiler sets m0 itself.  The s_nop covers what
-// the compiler, which does not look into the assembly, leaves open: the wait state between an SALU
-// write of m0 and the LDS DMA and, with NOP 4, the five between a VALU write of an SGPR (v_readlane:
-// a kernel short of SGPRs keeps bases in VGPR lanes) and a memory instruction that reads it.
-template <int NOP = 0>
+// wait_vm.  The LDS address is an m0 operand, so the compiler sets m0 itself.  It does not look into
+// the assembly for hazards: a memory instruction may not read an SGPR or m0 within five wait states
+// of a VALU instruction that wrote it (v_readlane, where a kernel short of SGPRs keeps bases in VGPR
+// lanes).  A scalar move may, and what it writes may be read at once, so both operands go through one
+// here; the second is also the wait state between a scalar write of m0 and the LDS DMA.
+// BARE: that wait state alone, for kernels whose assembly is checked to hold no such pair
+// (tests/test_lds_copy_wait_states.py).  The moves cost the kernels that wait on one chain of copies
+// and products 2 % (F16 4096 x 14336 at 9 rows 45.3 against 46.1 us, Q4_K 2048 x 8192 at 64 rows 37.1
+// against 38.0); five s_nop cost the int8 GEMMs 5 to 8 %.
+template <bool BARE = false>
 SYN_DEV void lds_dma16(uint32_t voff, const void* sbase, uint32_t lds) {
-    asm volatile("s_nop %3\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "{m0}"(lds), "n"(NOP)
-                 : "memory");
+    if constexpr (BARE) {
+        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :
+                     : "v"(voff), "s"(sbase), "{m0}"(lds)
+                     : "memory");
+    } else {
+        uint64_t base;
+        asm volatile("s_mov_b32 m0, m0\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0"
+                     : "=&s"(base)
+                     : "v"(voff), "s"(sbase), "{m0}"(lds)
+                     : "memory");
+    }
 }
 
 // The rows a launch computes: `rows`, or fewer when `active` points at a step descriptor's
@@ -413,11 +426,27 @@ SYN_DEV int active_rows(const uint32_t* active, int first, int rows) {
 }
 
 // 4 bytes per active lane from sbase + voff to LDS address lds + 4 * lane (as lds_dma16).
-template <int NOP = 0>
+template <bool BARE = false>
 SYN_DEV void lds_dma4(uint32_t voff, const void* sbase, uint32_t lds) {
-    asm volatile("s_nop %3\n\tglobal_load_lds_dword %0, %1"
+    if constexpr (BARE) {
+        asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1"
+                     :
+                     : "v"(voff), "s"(sbase), "{m0}"(lds)
+                     : "memory");
+    } else {
+        uint64_t base;
+        asm volatile("s_mov_b32 m0, m0\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dword %1, %0"
+                     : "=&s"(base)
+                     : "v"(voff), "s"(sbase), "{m0}"(lds)
+                     : "memory");
+    }
+}
+
+// As lds_dma16, from each lane's own address.
+SYN_DEV void lds_dma16_at(const void* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, m0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :
-                 : "v"(voff), "s"(sbase), "{m0}"(lds), "n"(NOP)
+                 : "v"(src), "{m0}"(lds)
                  : "memory");
 }
 

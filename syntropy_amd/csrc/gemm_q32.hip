@@ -218,14 +218,14 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
                 const int u = nth(i, C::WJ);
                 if constexpr (SPLIT) {
                     const uint32_t at = woff[i] + (uint32_t)C::STEP * (uint32_t)s;
-                    lds_dma16<4>(at < code_lim ? at : code_lim, g.w0, st + (uint32_t)(C::W_OFF + 1024 * u));
+                    lds_dma16(at < code_lim ? at : code_lim, g.w0, st + (uint32_t)(C::W_OFF + 1024 * u));
                 } else {
                     // an instruction's 64 pieces belong to one matrix
                     static_assert(C::R == 1 || C::ROWS * C::WCH % 64 == 0, "gate and up on whole copies");
                     const bool up = C::R == 2 && 64 * u >= C::ROWS * C::WCH;
                     const uint32_t at = (woff[i] + (uint32_t)C::STEP * (uint32_t)s) & ~15u;
                     const uint32_t lim = up ? wlast[C::R - 1] : wlast[0];
-                    lds_dma16<4>(at < lim ? at : lim, up ? wbase[C::R - 1] : wbase[0],
+                    lds_dma16(at < lim ? at : lim, up ? wbase[C::R - 1] : wbase[0],
                               st + (uint32_t)(C::W_OFF + 1024 * u));
                 }
             }
@@ -233,20 +233,20 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
 #pragma unroll
                 for (int i = 0; i < C::SPW; ++i) {
                     const uint32_t at = soff[i] + 8u * (uint32_t)s;
-                    lds_dma4<4>(at < scale_lim ? at : scale_lim, wscale, st + (uint32_t)(C::SC_OFF + 256 * nth(i, C::SJ)));
+                    lds_dma4(at < scale_lim ? at : scale_lim, wscale, st + (uint32_t)(C::SC_OFF + 256 * nth(i, C::SJ)));
                 }
             }
             // (a last stage past a row's end reads on into the next row, or the scales that follow
             // the codes: not used)
 #pragma unroll
             for (int i = 0; i < C::APW; ++i)
-                lds_dma16<4>(aoff[i], reinterpret_cast<const uint8_t*>(g.xq) + (size_t)(32 * G32_S) * (size_t)s,
+                lds_dma16(aoff[i], reinterpret_cast<const uint8_t*>(g.xq) + (size_t)(32 * G32_S) * (size_t)s,
                           st + (uint32_t)(C::A_OFF + 1024 * nth(i, C::AJ)));
 #pragma unroll
             for (int i = 0; i < C::DPW; ++i) {
                 const int u = nth(i, C::DJ);
                 const int b = G32_S * s + (64 * u + lane) / C::TOK;
-                lds_dma4<4>(4u * (doff[i] + (uint32_t)(b < nb ? b : nb - 1)), g.xd,
+                lds_dma4(4u * (doff[i] + (uint32_t)(b < nb ? b : nb - 1)), g.xd,
                          st + (uint32_t)(C::DX_OFF + 256 * u));
             }
         };

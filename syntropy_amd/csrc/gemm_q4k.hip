@@ -280,14 +280,14 @@ SYN_DEV void gemm_issue(const GemmSlots<MT>& s, const uint8_t* ab, const uint8_t
 #pragma unroll
     for (int i = 0; i < C::APW; ++i) {
         static_assert(GM_WAVES == 4, "16 tokens a round of copies");
-        lds_dma16(s.aoff ^ (64u * H), ab + 512u * (uint32_t)(16 * i < s.left ? 16 * i : s.left - 16),
+        lds_dma16<true>(s.aoff ^ (64u * H), ab + 512u * (uint32_t)(16 * i < s.left ? 16 * i : s.left - 16),
                   lds_addr(stage) + 1024u * (uint32_t)(wave + GM_WAVES * i));
     }
     if constexpr (H == 1) {
 #pragma unroll
         for (int i = 0; i < C::TPW; ++i) {
             const int u = wave + GM_WAVES * i;
-            if (64 * u + lane < C::TB / 16) lds_dma16(s.toff[i], tb, lds_addr(tail) + 1024u * (uint32_t)u);
+            if (64 * u + lane < C::TB / 16) lds_dma16<true>(s.toff[i], tb, lds_addr(tail) + 1024u * (uint32_t)u);
         }
     }
 }
@@ -792,12 +792,12 @@ __global__ __launch_bounds__(64 * GM_WAVES, 3) void k_moe_gemm(MoeGemmArgs g) {
             const uint32_t tl = lds_addr(tail);
 #pragma unroll
             for (int i = 0; i < C::APW; ++i)
-                lds_dma16(aoff[i] ^ (64u * H), ab, lds_addr(stage) + 1024u * (uint32_t)(wave + GM_WAVES * i));
+                lds_dma16<true>(aoff[i] ^ (64u * H), ab, lds_addr(stage) + 1024u * (uint32_t)(wave + GM_WAVES * i));
             if constexpr (H == 1) {
                 if (wave < 2)
-                    lds_dma16(sl.toff[0], tb, tl + 1024u * (uint32_t)wave);
+                    lds_dma16<true>(sl.toff[0], tb, tl + 1024u * (uint32_t)wave);
                 else
-                    lds_dma4(sl.toff[0], tb, tl + (wave == 2 ? 2048u : 2304u));
+                    lds_dma4<true>(sl.toff[0], tb, tl + (wave == 2 ? 2048u : 2304u));
             }
         }
     };

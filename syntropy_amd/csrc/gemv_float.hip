@@ -90,7 +90,7 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
             const int row = 4 * tr + (u & 3) < last ? 4 * tr + (u & 3) : last;
             if constexpr (VEC) {
                 const uint32_t at = 2u * KC * (uint32_t)sc + 16u * (uint32_t)(lane % (64 / G::RPC));
-                lds_dma16((uint32_t)row * rb + (at < rb ? at : rb - 16), wbase,
+                lds_dma16<true>((uint32_t)row * rb + (at < rb ? at : rb - 16), wbase,
                           lds_addr(st) + (uint32_t)(wave * G::WBYTES + u * G::WPIECE));
             } else {
                 const int e = KC * sc + 8 * (lane % (64 / G::RPC));
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
             const uint32_t dst = (uint32_t)((q / PR) * G::XROW + 1024 * (q % PR));
             if constexpr (VEC) {
                 const uint32_t at = 4u * KC * (uint32_t)sc + 1024u * (uint32_t)(q % PR) + 16u * (uint32_t)lane;
-                lds_dma16(at < 2 * rb ? at : 2 * rb - 16, x + (int64_t)t * k, lds_addr(xst) + dst);
+                lds_dma16<true>(at < 2 * rb ? at : 2 * rb - 16, x + (int64_t)t * k, lds_addr(xst) + dst);
             } else {
                 const int e = KC * sc + 256 * (q % PR) + 4 * lane;
                 const float* src = x + (int64_t)t * k;

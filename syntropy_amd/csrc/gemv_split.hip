@@ -691,9 +691,9 @@ __device__ __forceinline__ void qs_issue(const QsCopy* cp, uint32_t stage_lds, i
         const uint8_t* base = cp[u].base + (size_t)cp[u].step * (size_t)s;
         if (cp[u].on) {
             if (cp[u].wide)
-                lds_dma16(cp[u].voff, base, stage_lds + cp[u].lds);
+                lds_dma16<true>(cp[u].voff, base, stage_lds + cp[u].lds);
             else
-                lds_dma4(cp[u].voff, base, stage_lds + cp[u].lds);
+                lds_dma4<true>(cp[u].voff, base, stage_lds + cp[u].lds);
         }
     }
 }
@@ -890,7 +890,7 @@ __global__ __launch_bounds__(256) void k_gemm_q8_splitk(const uint8_t* __restric
         const uint32_t st = ring + (uint32_t)(C::STAGE * (s % QK_NS));
 #pragma unroll
         for (int u = 0; u < C::COP; ++u) {
-            if (u < ncop && cp[u].on) lds_dma16(cp[u].voff, cp[u].base + (size_t)cp[u].step * (size_t)s, st + cp[u].lds);
+            if (u < ncop && cp[u].on) lds_dma16<true>(cp[u].voff, cp[u].base + (size_t)cp[u].step * (size_t)s, st + cp[u].lds);
         }
     };
     float* terms = reinterpret_cast<float*>(lds + QK_NS * C::STAGE);

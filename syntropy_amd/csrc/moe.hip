@@ -865,19 +865,12 @@ SYN_DEV Slot make_slot(int s, const uint8_t* const (&bases)[C::NM], const ItemRo
     return r;
 }
 
-// The load is written as assembly so the compiler does not track it: it would otherwise wait
-// for every load into LDS still in flight before each LDS read, the next stages' included.
-// The explicit waits of the ring order the stages instead.
+// (The explicit waits of the ring order the stages.)
 SYN_DEV void issue_slot(const Slot& sl, int b, uint8_t* stage) {
     if (sl.live && sl.on) {
         const uint8_t* src = sl.x8 ? sl.src + x8_chunk_offset(sl.xg0 + (uint32_t)b, sl.xq, sl.xnb)
                                    : sl.src + (uint64_t)sl.step * (uint32_t)b;
-        const uint32_t dst = (uint32_t)(uintptr_t)(lds_ptr)(stage + sl.lds);
-        // the LDS address is an m0 operand (the compiler sets m0; s_nop is the wait state)
-        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                     :
-                     : "v"(src), "{m0}"(dst)
-                     : "memory");
+        lds_dma16_at(src, lds_addr(stage + sl.lds));
     }
 }
 
