@@ -16,7 +16,8 @@
 //   fma(dw * dx, M + s, -M * dw * dx) is then dw * dx * s rounded once, the reference's product, and
 //       one addition folds it.  (s = 0 gives +0.0 for either zero, which a sum from +0.0 does not
 //       see.)  An infinite scale (dw or dx past F16's range) makes that a NaN where the reference
-//       has an infinity, so an output that ends as NaN is computed again as written.
+//       may have an infinity, so a tile that ends with NaNs takes them again, as written, from its
+//       blocks whose scales are not finite (g32_settle).
 // Q4_0: the int8 operand holds 16 (n - 8) (a nibble in the high half of its byte, its top bit
 // flipped), and the scale is dw / 16: the same bound on s, the same exactness.
 //
@@ -102,26 +103,75 @@ struct G32Args {
     int top_k;
 };
 
-// Where block b of a row lies: its codes and its scale.
-template <int FMT, int SPLIT>
-SYN_DEV float g32_plain(const uint8_t* w, int n_out, int nb, int row, const int8_t* xq, const float* xd) {
-    constexpr int CB = FMT == T_Q8_0 ? 32 : 16;
-    float acc = 0.0f;
+// A 32 x 32 tile's outputs that ended as NaN, settled from the blocks whose weight or token scale is an
+// infinity or a NaN: the reference's terms (dw * dx) * s of those blocks alone.  Beside an infinite or
+// NaN term the finite ones (below 2^52 each) change nothing, and without one no output is a NaN.  The
+// wavefront looks at the scales 16 blocks at a time and stops where every NaN is known to stay one, so a
+// NaN row of activations costs a few blocks and any other scale at most one pass over the rows' scales,
+// whatever the number of NaNs: 4096 x 14336 Q8_0 at 64 rows 117 us, with a NaN row of activations 120,
+// with one infinite or NaN scale at a row's end 172 to 178 (the outputs one by one in their lanes:
+// 17300, 1340).
+// drow: the lane's row's first scale (dstep bytes a block), qrow: its code bytes (qstep); xq, xd: its
+// token's codes and scales.
+template <int FMT>
+SYN_DEV void g32_settle(v16f_q& acc, int nb, const uint8_t* drow, int dstep, const uint8_t* qrow, int qstep,
+                        const int8_t* xq, const float* xd) {
+    const int h = (threadIdx.x >> 5) & 1;
+    // bit 31 where v is a NaN, and bit 15 - i where v[i] is: no lane masks, of which a comparison each
+    // would take the scalar registers of the loop above
+    auto nan = [](float v) { return 0x7F800000u - (f2u(v) & 0x7FFFFFFFu); };
+    auto nans = [&](const v16f_q& v) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m = __builtin_amdgcn_alignbit(m, nan(v[i]), 31);
+        return m;
+    };
+    const uint32_t was = nans(acc);
+    if (__builtin_amdgcn_ballot_w64(was != 0) == 0) return;  // uniform
+    v16f_q sum = {};
+    bool more = true;
 #pragma unroll 1
-    for (int b = 0; b < nb; ++b) {
-        const uint64_t g = (uint64_t)row * nb + b;
-        const uint8_t* q = SPLIT ? w + g * CB : w + g * (CB + 2) + 2;
-        const uint16_t dw = SPLIT ? *reinterpret_cast<const uint16_t*>(w + (uint64_t)n_out * nb * CB + 2 * g)
-                                  : *reinterpret_cast<const uint16_t*>(q - 2);
-        int s = 0;
-#pragma unroll 1
-        for (int i = 0; i < 32; ++i) {
-            const int v = FMT == T_Q8_0 ? (int)(int8_t)q[i] : (int)((q[i & 15] >> (i & 16 ? 4 : 0)) & 15) - 8;
-            s += v * xq[32 * b + i];
+    for (int b0 = 0; more && b0 < nb; b0 += 16) {  // uniform
+        uint32_t odd = 0;  // bit j: block b0 + 8 h + j of the lane's row or token
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int b = b0 + 8 * h + j < nb ? b0 + 8 * h + j : nb - 1;
+            const uint32_t dw = *reinterpret_cast<const uint16_t*>(drow + (int64_t)b * dstep);
+            const uint32_t dx = f2u(xd[b]);
+            odd |= (dw & 0x7C00u) == 0x7C00u || (dx & 0x7F800000u) == 0x7F800000u ? 1u << j : 0u;
         }
-        acc = acc + (f16_to_f32(dw) * xd[b]) * (float)s;
+        uint32_t blocks = 0;  // any lane's
+#pragma unroll 1
+        for (int j = 0; j < 8; ++j) {
+            const uint64_t m = __builtin_amdgcn_ballot_w64((odd >> j & 1) != 0);
+            blocks |= ((uint32_t)m != 0 ? 1u << j : 0u) | ((uint32_t)(m >> 32) != 0 ? 256u << j : 0u);
+        }
+#pragma unroll 1
+        for (; more && blocks; blocks &= blocks - 1) {
+            const int b = b0 + __builtin_ctz(blocks);
+            if (b >= nb) break;  // (the last block again)
+            uint32_t w[4];
+            __builtin_memcpy(w, qrow + (int64_t)b * qstep + (FMT == T_Q8_0 ? 16 * h : 0), 16);
+            if constexpr (FMT == T_Q4_0) {  // 16 (n - 8), as the products take them
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] = ((w[i] << (h ? 0 : 4)) & 0xF0F0F0F0u) ^ 0x80808080u;
+            }
+            const v4i_q a = {(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+            const v4i_q x = *reinterpret_cast<const v4i_q*>(xq + 32 * (int64_t)b + 16 * h);
+            const float dw = f16_to_f32(*reinterpret_cast<const uint16_t*>(drow + (int64_t)b * dstep)) *
+                             (FMT == T_Q4_0 ? 0.0625f : 1.0f);
+            const v16i_q f = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, x, v16i_q{}, 0, 0, 0);
+            const v32f_q p = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, xd[b], v32f_q{}, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sum[i] = sum[i] + p[i] * (float)f[i];
+            more = __builtin_amdgcn_ballot_w64((was & ~nans(sum)) != 0) != 0;  // one is still open
+        }
     }
-    return acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t m = (uint32_t)((int32_t)nan(acc[i]) >> 31);
+        acc[i] = u2f((f2u(sum[i]) & m) | (f2u(acc[i]) & ~m));
+    }
 }
 
 template <int FMT, int SPLIT, int MODE, int RG, int TG, int TT>
@@ -385,6 +435,17 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
         else
             loop(std::integral_constant<int, 1>{});
         wait_vm<0>();  // the last (repeated) copies have landed
+        if (busy) {
+            const uint8_t* w = C::R == 2 && mat ? wm[C::R - 1] : wm[0];
+            const uint8_t* q = w + (uint64_t)rowc * rb + (SPLIT ? 0 : 2);
+            const uint8_t* d = SPLIT ? wscale + 2 * (uint64_t)rowc * (uint64_t)nb : q - 2;
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const uint64_t x = token(32 * (TT * tg + t) + c);
+                g32_settle<FMT>(acc[t], nb, d, SPLIT ? 2 : C::BB, q, SPLIT ? C::CB : C::BB, g.xq + x * (uint64_t)g.k,
+                                g.xd + x * (uint64_t)nb);
+            }
+        }
         if constexpr (MODE != G32_DENSE) lds_barrier();  // the last stages are read out
         v16f_q up[TT];
         if constexpr (MODE == G32_GATEUP) {  // [wavefront][tile][i][lane]
@@ -409,18 +470,9 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
             if (tt >= valid) continue;
             const int tk = t0 + tt;
             const int n0 = row0 + 32 * rg + 4 * h;
-            uint32_t nan = 0;
             float o[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                if constexpr (MODE == G32_GATEUP) {
-                    nan |= acc[t][i] != acc[t][i] || up[t][i] != up[t][i] ? 1u << i : 0u;
-                    o[i] = ref_silu(acc[t][i]) * up[t][i];
-                } else {
-                    nan |= acc[t][i] != acc[t][i] ? 1u << i : 0u;
-                    o[i] = acc[t][i];
-                }
-            }
+            for (int i = 0; i < 16; ++i) o[i] = MODE == G32_GATEUP ? ref_silu(acc[t][i]) * up[t][i] : acc[t][i];
             const uint64_t yrow = MODE == G32_DENSE ? (uint64_t)tk
                                   : MODE == G32_GATEUP ? (uint64_t)(e0 + (uint32_t)tk)
                                                        : (uint64_t)g.slots[e0 + (uint32_t)tk];
@@ -435,22 +487,6 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         if (n + i < g.n_out) yr[n + i] = o[4 * q + i];
-                }
-            }
-            if (nan) {  // a NaN or an infinite scale: these outputs as the reference writes them
-                const uint64_t xr = token(tt);
-#pragma unroll 1
-                for (; nan; nan &= nan - 1) {
-                    const int i = __builtin_ctz(nan);
-                    const int n = n0 + 8 * (i >> 2) + (i & 3);
-                    if (n >= g.n_out) continue;
-                    const int8_t* xq = g.xq + xr * (uint64_t)g.k;
-                    const float* xd = g.xd + xr * (uint64_t)nb;
-                    const float v = g32_plain<FMT, SPLIT>(wm[0], g.n_out, nb, n, xq, xd);
-                    if constexpr (MODE == G32_GATEUP)
-                        yr[n] = ref_silu(v) * g32_plain<FMT, SPLIT>(wm[C::R - 1], g.n_out, nb, n, xq, xd);
-                    else
-                        yr[n] = v;
                 }
             }
         }

@@ -91,6 +91,65 @@ def test_infinite_and_nan_scales(S, ty):
     check(S, ty, w.reshape(-1), n_out, k, x, rows, f"q32 ty={ty} infinite scales")
 
 
+@pytest.mark.parametrize("ty", [o.Q8_0, o.Q4_0])
+@pytest.mark.parametrize("rows,n_out,k", [(33, 40, 1056), (1025, 4099, 160)])  # one and two token tiles a wavefront
+def test_many_infinite_scales(S, ty, rows, n_out, k):
+    """Whole rows of infinite weight scales and activation scales, of one sign and of both, and infinities
+    in the last block of a partial stage and past the first 16 blocks."""
+    rs = np.random.default_rng(rows + 3)
+    nb = k // 32
+    w = blocks(rs, ty, n_out, k).reshape(n_out, nb, BYTES[ty])
+    f16 = lambda h: np.array([h], np.uint16).view(np.uint8)
+    w[0, :, :2] = f16(0x7C00)
+    w[1, ::2, :2], w[1, 1::2, :2] = f16(0x7C00), f16(0xFC00)
+    w[33, nb - 1, :2] = f16(0xFC00)
+    w[35, :, 2:] = 0x88  # sums of one sign (Q8_0) or zero (Q4_0): an infinity times zero
+    w[35, 1, :2] = f16(0x7C00)
+    w[38, nb // 2, :2] = f16(0x7E01)
+    x = rs.standard_normal((rows, k)).astype(np.float32)
+    x[1] *= 1e9
+    x[2] = np.abs(x[2]) * 1e9
+    x[rows - 1, k - 3] = -4e9
+    x[rows - 2, : 16 * 32 if nb > 16 else 64] = np.inf
+    check(S, ty, w.reshape(-1), n_out, k, x, rows, f"q32 ty={ty} many infinities {rows} {n_out}x{k}")
+
+
+@pytest.mark.parametrize("ty,split", [(o.Q8_0, False), (o.Q4_0, False), (o.Q8_0, True)])
+def test_nan_and_infinity_take_no_longer(S, ty, split):
+    """A NaN row of activations, an activation past the scales' range and an infinite weight scale, each
+    at the end of a row: at most one more pass over the rows' blocks (measured up to 1.5 times the call
+    without; the outputs one by one took 10 to 150 times it)."""
+    n_out, k, rows = 2048, 8192, 1024 if split else 64
+    rs = np.random.default_rng(29)
+    w = blocks(rs, ty, n_out, k)
+    x = rs.standard_normal((rows, k)).astype(np.float32)
+    y = torch.empty(rows, n_out, device="cuda")
+
+    def micros(w, x):
+        W = S.Weights(S.WeightType(ty), dev(w), n_out, k)
+        W, xd = S.repack(W) if split else W, dev(x)
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = float("inf")
+        for _ in range(5):
+            ev[0].record()
+            for _ in range(4):
+                S.gemv(W, xd, rows, y=y)
+            ev[1].record()
+            torch.cuda.synchronize()
+            best = min(best, 250 * ev[0].elapsed_time(ev[1]))
+        return best
+
+    announce(f"q32 ty={ty} split={split} time with NaNs")
+    clean = micros(w, x)
+    nan, big, winf = x.copy(), x.copy(), w.copy()
+    nan[3] = np.nan
+    big[3, -1] = 1e9
+    winf.reshape(n_out, k // 32, -1)[5, -1, :2] = np.array([0x7C00], np.uint16).view(np.uint8)
+    for what, t in (("NaN row", micros(w, nan)), ("infinite token scale", micros(w, big)),
+                    ("infinite weight scale", micros(winf, x))):
+        assert t < 4 * clean, f"{what}: {t:.0f} us against {clean:.0f}"
+
+
 @pytest.mark.parametrize("E,top_k,hidden,inter,rows,popular", [
     (4, 1, 160, 96, 300, 290),    # one expert's entries beyond the grid's tiles
     (3, 2, 64, 224, 70, 65), (6, 2, 288, 64, 90, 0), (16, 2, 96, 160, 33, 20), (1, 1, 32, 32, 129, 129)])
