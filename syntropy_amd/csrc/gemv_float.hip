@@ -48,8 +48,10 @@ struct GfCfg {
     static_assert(LDS <= 160 * 1024, "LDS");
 };
 
-// VEC: rows of whole 16-byte pieces at 16-byte aligned addresses, copied by global_load_lds; else
-// element by element through registers.
+// VEC: rows of whole 16-byte pieces at 16-byte aligned addresses.  Else a stage copies the KC elements'
+// space from the aligned piece that its first element lies in and takes KC - 32 of them, which leaves
+// every row's offset in its piece the same in all stages.  An aligned piece that holds a byte of a row
+// lies in the same page as that byte, so the reads around a row's ends stay on its pages.
 template <int BF16, int VEC, int C, int R, int WV, int KC, int NS>
 __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __restrict__ W, int n_out, int k,
                                                           const float* __restrict__ x, int rows,
@@ -60,14 +62,16 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
     rows = active_rows(active, 0, rows);
     // activation groups of the same weight rows run on the same XCD (workgroups go to the 8 XCDs
     // in turn), one after the other, so that the later ones find the weights in its L2
-    const int wb = groups == 1 ? (int)blockIdx.x : 8 * ((int)blockIdx.x / (8 * groups)) + (int)(blockIdx.x & 7);
-    const int t0 = groups == 1 ? 0 : 4 * C * (((int)blockIdx.x >> 3) % groups);
-    if (t0 >= rows) return;  // uniform
+    const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    const int wb = groups == 1 ? id : 8 * (id / (8 * groups)) + (id & 7);
+    const int t0 = groups == 1 ? 0 : 4 * C * ((id >> 3) % groups);
+    if (t0 >= rows || (int64_t)wb * WV * 4 * R >= n_out) return;  // uniform
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int b = lane >> 2, i = lane & 3;
     const int row0 = (wb * WV + wave) * 4 * R;
-    const int ns = (k + KC - 1) / KC;
+    constexpr int KS = VEC ? KC : KC - 32;  // elements a stage
+    const int ns = k / KS + (k % KS != 0);
     const uint32_t rb = 2u * (uint32_t)k;
     v4f_f acc[R][C][2];
 #pragma unroll
@@ -88,16 +92,21 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
         for (int u = 0; u < G::WCOPIES; ++u) {
             const int tr = G::RPC * (u / 4) + lane / (64 / G::RPC);
             const int row = 4 * tr + (u & 3) < last ? 4 * tr + (u & 3) : last;
+            const uint32_t to = lds_addr(st) + (uint32_t)(wave * G::WBYTES + u * G::WPIECE);
             if constexpr (VEC) {
                 const uint32_t at = 2u * KC * (uint32_t)sc + 16u * (uint32_t)(lane % (64 / G::RPC));
-                lds_dma16<true>((uint32_t)row * rb + (at < rb ? at : rb - 16), wbase,
-                          lds_addr(st) + (uint32_t)(wave * G::WBYTES + u * G::WPIECE));
+                lds_dma16<true>((uint32_t)row * rb + (at < rb ? at : rb - 16), wbase, to);
             } else {
-                const int e = KC * sc + 8 * (lane % (64 / G::RPC));
-                const uint16_t* src = reinterpret_cast<const uint16_t*>(wbase) + (int64_t)row * k;
-                uint16_t* dst = reinterpret_cast<uint16_t*>(st + wave * G::WBYTES + u * G::WPIECE) + 8 * lane;
-#pragma unroll
-                for (int q = 0; q < 8; ++q) dst[q] = e + q < k ? src[e + q] : (uint16_t)0;
+                // from the piece of the first of the copy's rows (two rows, of less than 2^25 bytes: 4
+                // rows apart)
+                const int r0 = 4 * G::RPC * (u / 4) + (u & 3) < last ? 4 * G::RPC * (u / 4) + (u & 3) : last;
+                const uint8_t* from = wbase + (uint64_t)r0 * rb;
+                const uint32_t mis = (uint32_t)((uintptr_t)from & 15);
+                const uint64_t at = 2ull * KS * (uint64_t)sc;
+                const uint32_t start = G::RPC == 1 ? mis : mis + (uint32_t)(row - r0) * rb;
+                const uint64_t end = (((uint64_t)start + rb - 1) & ~15ull) - (start & ~15u) - at;  // the row's last piece
+                const uint32_t off = 16u * (uint32_t)(lane % (64 / G::RPC));
+                lds_dma16<true>((start & ~15u) + (off < end ? off : (uint32_t)end), from - mis + at, to);
             }
         }
         uint8_t* xst = st + WV * G::WBYTES;
@@ -107,18 +116,31 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
             constexpr int PR = KC / 256;  // pieces of an activation row
             const int t = t0 + q / PR < rows ? t0 + q / PR : rows - 1;
             const uint32_t dst = (uint32_t)((q / PR) * G::XROW + 1024 * (q % PR));
+            const float* from = x + (int64_t)t * k;
             if constexpr (VEC) {
                 const uint32_t at = 4u * KC * (uint32_t)sc + 1024u * (uint32_t)(q % PR) + 16u * (uint32_t)lane;
-                lds_dma16<true>(at < 2 * rb ? at : 2 * rb - 16, x + (int64_t)t * k, lds_addr(xst) + dst);
+                lds_dma16<true>(at < 2 * rb ? at : 2 * rb - 16, from, lds_addr(xst) + dst);
             } else {
-                const int e = KC * sc + 256 * (q % PR) + 4 * lane;
-                const float* src = x + (int64_t)t * k;
-                float* d = reinterpret_cast<float*>(xst + dst) + 4 * lane;
-#pragma unroll
-                for (int z = 0; z < 4; ++z) d[z] = e + z < k ? src[e + z] : 0.0f;
+                const uint32_t mis = (uint32_t)((uintptr_t)from & 15);
+                const uint64_t at = 4ull * KS * (uint64_t)sc, end = ((mis + 2 * (uint64_t)rb - 1) & ~15ull) - at;
+                const uint32_t off = 1024u * (uint32_t)(q % PR) + 16u * (uint32_t)lane;
+                lds_dma16<true>(off < end ? off : (uint32_t)end, reinterpret_cast<const uint8_t*>(from) - mis + at,
+                                lds_addr(xst) + dst);
             }
         }
     };
+    // (not VEC) where the lane's rows start in their pieces
+    uint32_t woff[R], xoff[C];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int row = 4 * r + i < last ? 4 * r + i : last;
+        woff[r] = VEC ? 0u : (uint32_t)((uintptr_t)(wbase + (uint64_t)row * rb) & 15);
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int t = t0 + 4 * c + i < rows ? t0 + 4 * c + i : rows - 1;
+        xoff[c] = VEC ? 0u : (uint32_t)((uintptr_t)(x + (int64_t)t * k) & 15);
+    }
     auto cvt = [](uint32_t h) { return BF16 ? __builtin_bit_cast(float, h << 16) : f16_to_f32(h); };
     // `tail`: a stage that the row may end in; the others run without a branch, so that the LDS
     // reads of a step are issued under the products of the one before
@@ -127,29 +149,39 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
         const uint8_t* ws = st + wave * G::WBYTES + i * G::WPIECE + 4 * b;
         const uint8_t* xs = st + WV * G::WBYTES + i * G::XROW + 8 * b;
 #pragma unroll
-        for (int m = 0; m < G::MC; ++m) {
+        for (int m = 0; m < KS / 32; ++m) {
             float2 xb[C];
 #pragma unroll
-            for (int c = 0; c < C; ++c) xb[c] = *reinterpret_cast<const float2*>(xs + 4 * c * G::XROW + 128 * m);
+            for (int c = 0; c < C; ++c) {
+                const uint8_t* p = xs + 4 * c * G::XROW + 128 * m + xoff[c];
+                if constexpr (VEC)
+                    xb[c] = *reinterpret_cast<const float2*>(p);
+                else
+                    xb[c] = make_float2(reinterpret_cast<const float*>(p)[0], reinterpret_cast<const float*>(p)[1]);
+            }
             float a[R][2];
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                const uint32_t w = *reinterpret_cast<const uint32_t*>(ws + (r / G::RPC) * 4 * G::WPIECE +
-                                                                      (r % G::RPC) * 2 * KC + 64 * m);
+                const uint8_t* p = ws + (r / G::RPC) * 4 * G::WPIECE + (r % G::RPC) * 2 * KC + 64 * m + woff[r];
+                uint32_t w;
+                if constexpr (VEC)
+                    w = *reinterpret_cast<const uint32_t*>(p);
+                else
+                    w = reinterpret_cast<const uint16_t*>(p)[0] | (uint32_t)reinterpret_cast<const uint16_t*>(p)[1] << 16;
                 a[r][0] = cvt(w & 0xFFFFu);
                 a[r][1] = BF16 ? __builtin_bit_cast(float, w & 0xFFFF0000u) : cvt(w >> 16);
             }
             if constexpr (decltype(tail)::value) {  // elements past the row: 0 times -0.0, which no sum sees
-                const int e = KC * s + 32 * m + 2 * b;
+                const uint32_t e = (uint32_t)KS * (uint32_t)s + 32u * m + 2u * b, n = (uint32_t)k;
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
-                    a[r][0] = e < k ? a[r][0] : 0.0f;
-                    a[r][1] = e + 1 < k ? a[r][1] : 0.0f;
+                    a[r][0] = e < n ? a[r][0] : 0.0f;
+                    a[r][1] = e + 1 < n ? a[r][1] : 0.0f;
                 }
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
-                    xb[c].x = e < k ? xb[c].x : -0.0f;
-                    xb[c].y = e + 1 < k ? xb[c].y : -0.0f;
+                    xb[c].x = e < n ? xb[c].x : -0.0f;
+                    xb[c].y = e + 1 < n ? xb[c].y : -0.0f;
                 }
             }
 #pragma unroll
@@ -162,13 +194,13 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
         }
     };
     if (ns > 0) {
-        const int whole = k / KC;
+        const int whole = k / KS;
 #pragma unroll
         for (int s = 0; s < NS - 1; ++s) issue(s);
         for (int s = 0; s < ns; ++s) {
             // stage s has landed (the NS - 2 after it may fly), the previous one is read out, and the
             // next copies go into its place
-            wait_vm<VEC ? G::COPIES * (NS - 2) : 0>();
+            wait_vm<G::COPIES * (NS - 2)>();
             lds_barrier();
             issue(s + NS - 1);
             if (s < whole)
@@ -205,6 +237,8 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
         }
 }
 
+constexpr int64_t GF_MAX_X = 1 << 20;
+
 template <int BF16, int VEC, int C, int R, int WV, int KC, int NS>
 static void launch_float(const uint8_t* W, int n_out, int k, const float* x, int rows, float* y, hipStream_t stream,
                          const uint32_t* active) {
@@ -216,8 +250,10 @@ static void launch_float(const uint8_t* W, int n_out, int k, const float* x, int
     static const hipError_t attr = hipFuncSetAttribute((const void*)k_gemv_float<BF16, VEC, C, R, WV, KC, NS>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)G::LDS);
     (void)attr;
-    hipLaunchKernelGGL((k_gemv_float<BF16, VEC, C, R, WV, KC, NS>), dim3((unsigned)wgs), dim3(64 * WV), G::LDS, stream,
-                       W, n_out, k, x, rows, y, active, groups);
+    // a dimension of the grid holds less than 2^32 threads: whole rounds of the XCDs in x, the rest in y
+    const dim3 grid((unsigned)(wgs < GF_MAX_X ? wgs : GF_MAX_X), (unsigned)((wgs + GF_MAX_X - 1) / GF_MAX_X));
+    hipLaunchKernelGGL((k_gemv_float<BF16, VEC, C, R, WV, KC, NS>), grid, dim3(64 * WV), G::LDS, stream, W, n_out, k, x,
+                       rows, y, active, groups);
 }
 
 // Workgroups of 64 weight rows (eight wavefronts of eight) from this many of them on, else of
@@ -227,27 +263,34 @@ constexpr int GF_WIDE_WGS = 129;
 
 // Beyond 16 activation rows, groups of 16 (32 in one workgroup leave one wavefront a SIMD: 32064 x
 // 4096 at 32 rows 192 us against 174).
+template <int BF16, int VEC>
+static void launch_float_rows(const uint8_t* W, int n_out, int k, const float* x, int rows, float* y,
+                              hipStream_t stream, const uint32_t* active) {
+    // (rows of 2^24 elements and more: a copy within one row, whose offsets then fit 32 bits)
+    const bool wide = k <= (1 << 24) && (int64_t)((n_out + 63) / 64) * ((rows + 15) / 16) >= GF_WIDE_WGS;
+    if (rows <= 4 && wide)
+        launch_float<BF16, VEC, 1, 2, 8, 256, 4>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 4)
+        launch_float<BF16, VEC, 1, 1, 4, 512, 4>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 8 && wide)
+        launch_float<BF16, VEC, 2, 2, 8, 256, 3>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 8)
+        launch_float<BF16, VEC, 2, 1, 4, 512, 4>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 12 && wide)
+        launch_float<BF16, VEC, 3, 2, 8, 256, 3>(W, n_out, k, x, rows, y, stream, active);
+    else if (wide)
+        launch_float<BF16, VEC, 4, 2, 8, 256, 3>(W, n_out, k, x, rows, y, stream, active);
+    else
+        launch_float<BF16, VEC, 4, 1, 4, 512, 3>(W, n_out, k, x, rows, y, stream, active);
+}
+
 template <int BF16>
 static void launch_float_fmt(const uint8_t* W, int n_out, int k, const float* x, int rows, float* y,
                              hipStream_t stream, const uint32_t* active) {
-    const bool vec = k % 8 == 0 && k <= (1 << 24) && ((uintptr_t)W & 15) == 0 && ((uintptr_t)x & 15) == 0;
-    const bool wide = (int64_t)((n_out + 63) / 64) * ((rows + 15) / 16) >= GF_WIDE_WGS;
-    if (!vec)
-        launch_float<BF16, 0, 4, 1, 4, 512, 2>(W, n_out, k, x, rows, y, stream, active);
-    else if (rows <= 4 && wide)
-        launch_float<BF16, 1, 1, 2, 8, 256, 4>(W, n_out, k, x, rows, y, stream, active);
-    else if (rows <= 4)
-        launch_float<BF16, 1, 1, 1, 4, 512, 4>(W, n_out, k, x, rows, y, stream, active);
-    else if (rows <= 8 && wide)
-        launch_float<BF16, 1, 2, 2, 8, 256, 3>(W, n_out, k, x, rows, y, stream, active);
-    else if (rows <= 8)
-        launch_float<BF16, 1, 2, 1, 4, 512, 4>(W, n_out, k, x, rows, y, stream, active);
-    else if (rows <= 12 && wide)
-        launch_float<BF16, 1, 3, 2, 8, 256, 3>(W, n_out, k, x, rows, y, stream, active);
-    else if (wide)
-        launch_float<BF16, 1, 4, 2, 8, 256, 3>(W, n_out, k, x, rows, y, stream, active);
+    if (k % 8 == 0 && k <= (1 << 24) && ((uintptr_t)W & 15) == 0 && ((uintptr_t)x & 15) == 0)
+        launch_float_rows<BF16, 1>(W, n_out, k, x, rows, y, stream, active);
     else
-        launch_float<BF16, 1, 4, 1, 4, 512, 3>(W, n_out, k, x, rows, y, stream, active);
+        launch_float_rows<BF16, 0>(W, n_out, k, x, rows, y, stream, active);
 }
 
 void launch_gemv_float(int ty, const uint8_t* W, int n_out, int k, const float* x, int rows, float* y,

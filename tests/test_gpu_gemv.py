@@ -408,6 +408,39 @@ def test_float_gemv_tiles(S, ty, rows, n_out, k, scale):
     assert_same(got, o.gemv(ty, w, n_out, k, x, rows, threads=8), f"ty {ty}")
 
 
+@pytest.mark.parametrize("ty", [o.F16, o.BF16])
+@pytest.mark.parametrize("rows,n_out,k,w_at,x_at", [
+    (1, 33, 1, 2, 4), (2, 70, 481, 0, 0), (4, 17, 1441, 6, 12), (7, 40, 960, 14, 0), (16, 21, 512, 0, 8),
+    (20, 35, 1023, 2, 4), (3, 8300, 225, 10, 4), (6, 8257, 449, 0, 0), (12, 8193, 672, 2, 12), (17, 4200, 37, 4, 4)])
+def test_float_gemv_any_address(S, ty, rows, n_out, k, w_at, x_at):
+    """Rows of any length at any even (weights) and 4-byte (activations) address: windows of 480 and 224
+    elements and their edges, both row widths, guard bytes around the operands that no value may see."""
+    rng = GemvRng(ty + rows * 3 + k)
+    w = gemv_weights(rng, ty, n_out, k, o.f16_bits, o.round_bf16)
+    x = gemv_activations(rng, rows, k).astype(np.float32)
+    wb = torch.full((w.size + 64,), 0xFF, dtype=torch.uint8, device="cuda")  # NaNs
+    wb[16 + w_at:16 + w_at + w.size] = dev(w)
+    xb = torch.full((rows * k + 16,), float("nan"), device="cuda")
+    xb[4 + x_at // 4:4 + x_at // 4 + rows * k] = dev(x).reshape(-1)
+    announce(f"float gemv ty={ty} rows={rows} {n_out}x{k} at {w_at}, {x_at}")
+    got = host(S.gemv(S.Weights(S.WeightType(ty), wb[16 + w_at:16 + w_at + w.size], n_out, k),
+                      xb[4 + x_at // 4:4 + x_at // 4 + rows * k].view(rows, k), rows))
+    assert_same(got, o.gemv(ty, w, n_out, k, x, rows, threads=8), f"ty {ty}")
+
+
+def test_float_gemv_rows_past_a_grid_dimension(S):
+    """More activation rows than a grid of one dimension has threads for."""
+    rows, n_out, k = (1 << 24) + 21, 64, 8
+    rng = GemvRng(77)
+    w = gemv_weights(rng, o.F16, n_out, k, o.f16_bits, o.round_bf16)
+    x = torch.randn(rows, k, device="cuda", generator=torch.Generator("cuda").manual_seed(3))
+    announce(f"float gemv rows={rows} {n_out}x{k}")
+    y = S.gemv(S.Weights(S.WeightType.F16, dev(w), n_out, k), x, rows)
+    at = torch.tensor([0, 15, 16, 17, 4095, 1 << 20, (1 << 23) + 5, (1 << 24) - 1, 1 << 24, rows - 6, rows - 1], device="cuda")
+    want = o.gemv(o.F16, w, n_out, k, host(x[at]), len(at), threads=1)
+    assert_same(host(y[at]), want, "sampled rows")
+
+
 def test_float_gemv_golden_case(S):
     """The pinned output bits of crates/kernels-cpu/src/gemv/tests.rs:726-777 on the device."""
     from test_oracle_pins import PINNED
