@@ -87,7 +87,10 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
     const int last = n_out - 1 - (row0 < n_out ? row0 : n_out - 1);  // the last row, from wbase
     auto issue = [&](int s) {
         uint8_t* st = lds + (s % NS) * G::STAGE;
-        const int sc = s < ns ? s : ns - 1;  // a stage past the row repeats the last, so that the counts stay
+        // a stage past the row: of two, none flies but the next (the wait is for all); of more, the last
+        // again, so that the counts stay
+        if (NS == 2 && s >= ns) return;
+        const int sc = s < ns ? s : ns - 1;
 #pragma unroll
         for (int u = 0; u < G::WCOPIES; ++u) {
             const int tr = G::RPC * (u / 4) + lane / (64 / G::RPC);
@@ -150,6 +153,7 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
         const uint8_t* xs = st + WV * G::WBYTES + i * G::XROW + 8 * b;
 #pragma unroll
         for (int m = 0; m < KS / 32; ++m) {
+            if (decltype(tail)::value && KS * s + 32 * m >= k) break;  // uniform
             float2 xb[C];
 #pragma unroll
             for (int c = 0; c < C; ++c) {
@@ -211,29 +215,32 @@ __global__ __launch_bounds__(64 * WV, 1) void k_gemv_float(const uint8_t* __rest
         wait_vm<0>();  // the last (repeated) copies have landed before the workgroup ends
     }
     // the halving fold: accumulators 2 b + j and 16 on (block b + 8), 8 on (b + 4), 4 on (b + 2),
-    // 2 on (b + 1), then the lane's own two; block 0 (lanes 0 to 3) ends with the sums
+    // 2 on (b + 1), then the lane's own two.  The first two steps take two and then four of the tile's
+    // rows at once, each half or quarter of the lanes another row, so that a tile's 16 sums end in a
+    // lane each: lanes 16 p + i hold activation row i of weight row 0, 2, 1, 3 for p = 0 to 3.
+    const int q = (lane >> 3 & 2) | (lane >> 5);
+    auto halves = [](float a, float b) __attribute__((always_inline)) {
+        const auto v = __builtin_amdgcn_permlane32_swap(f2u(a), f2u(b), false, false);
+        return u2f(v[0]) + u2f(v[1]);
+    };
+    auto quarters = [](float a, float b) __attribute__((always_inline)) {
+        const auto v = __builtin_amdgcn_permlane16_swap(f2u(a), f2u(b), false, false);
+        return u2f(v[0]) + u2f(v[1]);
+    };
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            const int t = t0 + 4 * c + i;
+            float v[2];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                float v[2];
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    uint32_t u = f2u(acc[r][c][j][q]);
-                    const auto h16 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-                    u = f2u(u2f(h16[0]) + u2f(h16[1]));
-                    const auto h8 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-                    float f = u2f(h8[0]) + u2f(h8[1]);
-                    f = f + u2f(dpp_u32<0x108>(f2u(f)));  // row_shl:8
-                    f = f + u2f(dpp_u32<0x104>(f2u(f)));  // row_shl:4
-                    v[j] = f;
-                }
-                const int row = row0 + 4 * r + q;
-                if (lane < 4 && t < rows && row < n_out) y[(int64_t)t * n_out + row] = v[0] + v[1];
+            for (int j = 0; j < 2; ++j) {
+                const v4f_f a = acc[r][c][j];
+                float f = quarters(halves(a[0], a[1]), halves(a[2], a[3]));
+                f = f + u2f(dpp_u32<0x128>(f2u(f)));  // row_ror:8
+                v[j] = f + u2f(dpp_u32<0x124>(f2u(f)));  // row_ror:4
             }
+            const int t = t0 + 4 * c + i, row = row0 + 4 * r + q;
+            if ((lane & 12) == 0 && t < rows && row < n_out) y[(int64_t)t * n_out + row] = v[0] + v[1];
         }
 }
 
@@ -261,6 +268,14 @@ static void launch_float(const uint8_t* W, int n_out, int k, const float* x, int
 // 24.3 us in 224 workgroups against 33.6 in 896, 4096 x 4096 at 24 rows 36 us in 128 against 33.
 constexpr int GF_WIDE_WGS = 129;
 
+// Short rows have few stages to hide a workgroup's first copies and its fold behind: they take two stages
+// a ring and half the wavefronts, so that a CU holds several workgroups and one starts while another
+// ends.  Up to four activation rows, rows of medium length too are better off with two workgroups of two
+// stages than with one of four.  Four stages of eight wavefronts | two of eight | two of four: one row of
+// 50000 x 768 21 | 16 | 15 us, 50000 x 2048 35 | 35 | 38, 32064 x 4096 46 | 43 | 52, 14336 x 14336 86 | 90 | 83;
+// 16 rows of 50000 x 768 38 | 35 | 30, 50000 x 4096 137 | 135 | 126.
+constexpr int GF_SHORT = 1024, GF_MID = 4096;
+
 // Beyond 16 activation rows, groups of 16 (32 in one workgroup leave one wavefront a SIMD: 32064 x
 // 4096 at 32 rows 192 us against 174).
 template <int BF16, int VEC>
@@ -268,7 +283,18 @@ static void launch_float_rows(const uint8_t* W, int n_out, int k, const float* x
                               hipStream_t stream, const uint32_t* active) {
     // (rows of 2^24 elements and more: a copy within one row, whose offsets then fit 32 bits)
     const bool wide = k <= (1 << 24) && (int64_t)((n_out + 63) / 64) * ((rows + 15) / 16) >= GF_WIDE_WGS;
-    if (rows <= 4 && wide)
+    if (wide && k <= GF_SHORT) {
+        if (rows <= 4)
+            launch_float<BF16, VEC, 1, 2, 4, 256, 2>(W, n_out, k, x, rows, y, stream, active);
+        else if (rows <= 8)
+            launch_float<BF16, VEC, 2, 2, 4, 256, 2>(W, n_out, k, x, rows, y, stream, active);
+        else if (rows <= 12)
+            launch_float<BF16, VEC, 3, 2, 4, 256, 2>(W, n_out, k, x, rows, y, stream, active);
+        else
+            launch_float<BF16, VEC, 4, 2, 4, 256, 2>(W, n_out, k, x, rows, y, stream, active);
+    } else if (rows <= 4 && wide && k <= GF_MID)
+        launch_float<BF16, VEC, 1, 2, 8, 256, 2>(W, n_out, k, x, rows, y, stream, active);
+    else if (rows <= 4 && wide)
         launch_float<BF16, VEC, 1, 2, 8, 256, 4>(W, n_out, k, x, rows, y, stream, active);
     else if (rows <= 4)
         launch_float<BF16, VEC, 1, 1, 4, 512, 4>(W, n_out, k, x, rows, y, stream, active);

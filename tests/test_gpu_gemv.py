@@ -410,14 +410,16 @@ def test_float_gemv_tiles(S, ty, rows, n_out, k, scale):
 
 @pytest.mark.parametrize("ty", [o.F16, o.BF16])
 @pytest.mark.parametrize("rows,n_out,k,w_at,x_at", [
-    (1, 33, 1, 2, 4), (2, 70, 481, 0, 0), (4, 17, 1441, 6, 12), (7, 40, 960, 14, 0), (16, 21, 512, 0, 8),
+    (1, 8200, 1024, 0, 0), (7, 8193, 8, 0, 0), (11, 8207, 1016, 0, 0), (20, 4100, 264, 0, 0), (4, 8300, 1032, 0, 0),
+    (2, 8200, 4104, 0, 0), (1, 33, 1, 2, 4), (2, 70, 481, 0, 0), (4, 17, 1441, 6, 12), (7, 40, 960, 14, 0), (16, 21, 512, 0, 8),
     (20, 35, 1023, 2, 4), (3, 8300, 225, 10, 4), (6, 8257, 449, 0, 0), (12, 8193, 672, 2, 12), (17, 4200, 37, 4, 4)])
 def test_float_gemv_any_address(S, ty, rows, n_out, k, w_at, x_at):
     """Rows of any length at any even (weights) and 4-byte (activations) address: windows of 480 and 224
     elements and their edges, both row widths, guard bytes around the operands that no value may see."""
-    rng = GemvRng(ty + rows * 3 + k)
-    w = gemv_weights(rng, ty, n_out, k, o.f16_bits, o.round_bf16)
-    x = gemv_activations(rng, rows, k).astype(np.float32)
+    rs = np.random.default_rng(rows * 3 + k)
+    w = rs.standard_normal(n_out * k).astype(np.float32)
+    w = (w.astype(np.float16) if ty == o.F16 else (w.view(np.uint32) >> 16).astype(np.uint16)).view(np.uint8)
+    x = rs.standard_normal((rows, k)).astype(np.float32)
     wb = torch.full((w.size + 64,), 0xFF, dtype=torch.uint8, device="cuda")  # NaNs
     wb[16 + w_at:16 + w_at + w.size] = dev(w)
     xb = torch.full((rows * k + 16,), float("nan"), device="cuda")
