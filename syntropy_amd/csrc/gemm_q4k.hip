@@ -203,7 +203,9 @@ struct GemmArgs {
     float* y;
     int N, T, nb, tpad;
     uint32_t rb;  // weight row bytes
-    int xcd_tokens;  // token tiles an XCD takes (a 1-D grid), or 0: blockIdx.x, blockIdx.y the row and token tiles
+    // blockIdx.x, blockIdx.y are the row and token tiles or, in a 1-D grid,
+    int xcd_tokens;  // not 0: an XCD takes this many token tiles;
+    int row_tiles;   // not 0: whole eights of row tiles come first, token tile by token tile, then the other rows
     const uint32_t* active;  // a step descriptor's rows_active, or null
 };
 
@@ -482,9 +484,16 @@ __global__ __launch_bounds__(64 * GM_WAVES, 2) void k_gemm_q4k(GemmArgs g) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: copy bases in SGPRs
     const int c = lane & 15, p = lane >> 4;
-    const int per = g.xcd_tokens, id = (int)blockIdx.x >> 3;
-    const int nx = per ? id / per : (int)blockIdx.x;
-    const int ty = per ? ((int)blockIdx.x & 7) * per + id - nx * per : (int)blockIdx.y;
+    int nx = (int)blockIdx.x, ty = (int)blockIdx.y;
+    if (g.xcd_tokens) {
+        const int id = nx >> 3;
+        ty = (nx & 7) * g.xcd_tokens + id % g.xcd_tokens, nx = id / g.xcd_tokens;
+    } else if (g.row_tiles) {
+        const int eights = g.row_tiles & ~7, first = eights * ((g.T + C::TT - 1) / C::TT);
+        const bool rest = nx >= first;
+        const int id = rest ? nx - first : nx, wide = rest ? g.row_tiles - eights : eights;
+        ty = id / wide, nx = (rest ? eights : 0) + id % wide;
+    }
     const int cols = GU ? g.N / 2 : g.N;
     const int n0 = GU ? nx * (gemm_rows(NT) / 2) + 16 * wave : nx * gemm_rows(NT) + 16 * NT * wave, t0 = ty * C::TT;
     const int T = active_rows(g.active, 0, g.T);
@@ -567,7 +576,14 @@ static void launch_gemm_tiles(GemmArgs g, hipStream_t stream) {
     // against 400).
     g.xcd_tokens = g.layout != LAYOUT_X8 && ny % 8 == 0 && nx < (1u << 23) / ny &&
                            (int64_t)g.T * 512 > (int64_t)g.N * 144 ? (int)(ny / 8) : 0;
-    const dim3 grid(g.xcd_tokens ? nx * ny : nx, g.xcd_tokens ? 1u : ny);
+    // Where the row tiles are no multiple of 8, a row's tile goes to another XCD at every token tile, and
+    // each L2 sees all weights.  In X8, whose lines are read eight times, that took up to four times as
+    // long (6000 x 4096, 47 tiles: 144 us at 600 rows, 285 at 2048; 14000 x 4096, 110 tiles: 323 at 1024),
+    // so the odd tiles go last (74, 181, 216); up to 16 tiles they are too large a part (14 tiles of 8192: 148
+    // against 154 us).  GGUF order does not need it (within 2 %).
+    g.row_tiles = g.layout == LAYOUT_X8 && nx % 8 != 0 && nx > 16 && nx < (1u << 23) / ny ? (int)nx : 0;
+    const bool flat = g.xcd_tokens || g.row_tiles;
+    const dim3 grid(flat ? nx * ny : nx, flat ? 1u : ny);
     hipLaunchKernelGGL((k_gemm_q4k<HALVES, MT, NT, GU>), grid, dim3(64 * GM_WAVES), C::template LDS<HALVES>, stream, g);
 }
 
