@@ -882,7 +882,7 @@ int syn_gate_up_act_rows(uint32_t layout, int32_t wtype, const void* w, uint64_t
     // not take, a refused call among that, goes on below)
     if ((layout == SYN_LAYOUT_SOURCE || (layout == SYN_LAYOUT_X8 && k_in % 2048 == 0)) &&
         use_gemm(wtype, rows, 2 * n_out, k_in) && w && x && aligned(w, 16) && aligned(x, 16) &&
-        w_bytes >= 2ull * n_out * (k_in / 256) * 144 && syn::gemm_q4k_gate_up_fits((int)layout, (int)n_out, (int)rows)) {
+        w_bytes >= 2ull * n_out * (k_in / 256) * 144 && syn::gemm_q4k_gate_up_fits((int)n_out, (int)rows)) {
         const syn::GemmAct a = syn::gemm_act_at((uint8_t*)ws, (int64_t)gemm_tpad(rows), (int)k_in);
         syn::launch_gemm_act(x, (int)rows, (int)k_in, a, (hipStream_t)stream, active);
         if (int rc = check_launch(W)) return rc;

@@ -546,18 +546,31 @@ bool gemm_q4k_supported(int n_out, int k) {
 // The wavefront tile.  A large one makes each weight operand once for more tokens and reads each token
 // once for more rows, a small one gives the SIMDs wavefronts: one alone issues a vector operation
 // every five cycles, two every two and a half.  Microseconds measured for 32 tokens x 16 rows | 64 x
-// 16 | 64 x 32 (whole super-blocks, halves) | 128 x 32, X8:
-//   4096 x 4096 at 64 rows (512 wavefronts of 32 x 16)   21 | 27 | 45, 44 | 48
-//   4096 x 4096 at 200 (1792)                            34 | 35 | 50, 49 | 75
-//   4096 x 4096 at 333 (2816; 1536 of 64 x 16)           53 | 47 | 54, 52 | 78
-//   14336 x 4096 at 200 (3584 of 64 x 16)               104 | 85 | 70, 80 | 82
-//   14336 x 4096 at 333 (336 workgroups of 128 x 128)   154 | 127 | 112, 110 | 97
-//   14336 x 4096 at 1024 (896)                          424 | 314 | 246, 255 | 215
+// 16 | 64 x 32 (whole super-blocks, halves) | 128 x 32:
+//                                                        X8                          GGUF
+//   4096 x 4096 at 64 rows (512 wavefronts of 32 x 16)   21 | 27 | 45, 44 | 48       22 | 28 | 43, 42 | 47
+//   4096 x 4096 at 200 (1792)                            34 | 35 | 50, 49 | 75       29 | 32 | 46, 45 | 73
+//   4096 x 4096 at 333 (1536 of 64 x 16)                 53 | 47 | 54, 52 | 78       40 | 41 | 48, 47 | 75
+//   8192 x 2048 at 333 (3072)                                                        34 | 32 | 36, 36 | 42
+//   14336 x 4096 at 200 (3584)                          104 | 85 | 70, 80 | 82       71 | 62 | 59, 62 | 74
+//   8192 x 2048 at 448 (3584)                                                        41 | 39 | 37, 36 | 43
+//   14336 x 4096 at 333 (336 workgroups of 128 x 128)   154 | 127 | 112, 110 | 97    96 | 89 | 93, 81 | 80
+//   11264 x 2048 at 512 (352)                                                        57 | 52 | 51, 47 | 54
+//   11264 x 2048 at 600 (440)                                                        68 | 59 | 60, 59 | 55
+//   14336 x 4096 at 600 (560)                          255 | 192 | 160, 161 | 155   160 | 136 | 127, 120 | 140
+//   14336 x 4096 at 1024 (896)                          424 | 314 | 246, 255 | 215   258 | 218 | 204, 181 | 187
+//   4096 x 4096 at 2048 (512)                                                       153 | 133 | 119, 117 | 108
+//   14336 x 4096 at 2048 (1792)                         878 | 639 | 487, 497 | 388   514 | 425 | 386, 346 | 332
 // X8 reaches the 128-token form first: a 16-byte chunk of a block shares its 128-byte line with seven
 // other blocks' chunks, so a workgroup draws eight times its weight bytes through its L1, and twice
-// the tokens halve that (GGUF at 512 rows, 448 workgroups: 113 against 119 with 64 x 32; at 333: 90 against 89).  64 x 32 with whole super-blocks holds two workgroups a CU, halves three: the former
-// while two hold them all.
-constexpr int64_t GM_SMALL_WAVES = 2048, GM_MID_WAVES = 3072, GM_WIDE_X8 = 320, GM_WIDE = 448;
+// the tokens halve that.  The 128-token form holds 512 workgroups on the chip, the 64-token one 768; in
+// GGUF order it is the better one where its last round is nearly full or one of several.  64 x 32 with whole
+// super-blocks holds two workgroups a CU, halves three: the former while two hold them all.
+// Against eight wavefronts of 64 x 32 a CU, whose weights went through LDS, GGUF order is up to 7 % slower where
+// that form's 256 workgroups just filled the chip (4096 x 14336 at 850 rows 202 against 189 us, 8192 x 2048
+// at 448 36.5 against 35.2; eight wavefronts with the weights in registers are no faster).
+constexpr int64_t GM_SMALL_WAVES = 2048, GM_MID_WAVES = 3072, GM_WIDE_X8 = 320, GM_WIDE = 420;
+constexpr int64_t GM_WIDE_ROUND = 512, GM_WIDE_NEXT = 896;
 
 template <bool HALVES, int MT, int NT, bool GU = false>
 static void launch_gemm_tiles(GemmArgs g, hipStream_t stream) {
@@ -604,14 +617,14 @@ static GemmArgs gemm_args(int layout, const uint8_t* W, int n_out, int k, GemmAc
     return g;
 }
 
-static bool gemm_mid(int layout, int64_t n, int64_t t) {
-    return (n + 15) / 16 * ((t + 63) / 64) <= (layout == LAYOUT_X8 ? GM_MID_WAVES : GM_MID_WAVES + 512);
-}
+static bool gemm_mid(int64_t n, int64_t t) { return (n + 15) / 16 * ((t + 63) / 64) <= GM_MID_WAVES; }
 
 template <bool GU>
 static void launch_gemm_wide(const GemmArgs& g, hipStream_t stream) {
     const int64_t n = g.N, t = g.T;
-    if ((n + 127) / 128 * ((t + 127) / 128) >= (g.layout == LAYOUT_X8 ? GM_WIDE_X8 : GM_WIDE))
+    const int64_t wide = (n + 127) / 128 * ((t + 127) / 128);  // workgroups of 128 tokens
+    if (g.layout == LAYOUT_X8 ? wide >= GM_WIDE_X8
+                              : wide >= GM_WIDE_NEXT || (wide >= GM_WIDE && wide <= GM_WIDE_ROUND))
         launch_gemm_tiles<true, 8, 2, GU>(g, stream);
     else if ((n + 127) / 128 * ((t + 63) / 64) <= 512)
         launch_gemm_tiles<false, 4, 2, GU>(g, stream);
@@ -625,7 +638,7 @@ void launch_gemm_q4k(int layout, const uint8_t* W, int n_out, int k, GemmAct a, 
     const int64_t n = n_out, t = T;
     if ((n + 15) / 16 * ((t + 31) / 32) <= GM_SMALL_WAVES)
         launch_gemm_tiles<false, 2, 1>(g, stream);
-    else if (gemm_mid(layout, n, t))
+    else if (gemm_mid(n, t))
         launch_gemm_tiles<true, 4, 1>(g, stream);
     else
         launch_gemm_wide<false>(g, stream);
@@ -634,9 +647,9 @@ void launch_gemm_q4k(int layout, const uint8_t* W, int n_out, int k, GemmAct a, 
 // Where the product takes tiles of two 16-row tiles a wavefront: GateUpAct's gate and up then meet in
 // one (no [T][2 n] product written and read back: 5632 x 2048 at 333 rows 43.1 -> 38.8 us); below, the
 // smaller tiles and k_silu_mul.
-bool gemm_q4k_gate_up_fits(int layout, int n, int T) {
+bool gemm_q4k_gate_up_fits(int n, int T) {
     const int64_t n2 = 2 * (int64_t)n;
-    return (n2 + 15) / 16 * ((T + 31) / 32) > GM_SMALL_WAVES && !gemm_mid(layout, n2, T);
+    return (n2 + 15) / 16 * ((T + 31) / 32) > GM_SMALL_WAVES && !gemm_mid(n2, T);
 }
 
 void launch_gemm_q4k_gate_up(int layout, const uint8_t* W, int n, int k, GemmAct a, int T, float* y,

@@ -165,7 +165,7 @@ bool gemm_q4k_supported(int n_out, int k);
 void launch_gemm_q4k(int layout, const uint8_t* W, int n_out, int k, GemmAct a, int T, float* y, hipStream_t stream,
                      const uint32_t* active = nullptr);
 // GateUpAct{Silu} of a stacked [gate; up] matrix of 2 n rows, where gemm_q4k_gate_up_fits
-bool gemm_q4k_gate_up_fits(int layout, int n, int T);
+bool gemm_q4k_gate_up_fits(int n, int T);
 void launch_gemm_q4k_gate_up(int layout, const uint8_t* W, int n, int k, GemmAct a, int T, float* y,
                              hipStream_t stream, const uint32_t* active = nullptr);
 // The MoE expert FFN at many tokens on the same kernels: entries padded to 64-entry tiles per

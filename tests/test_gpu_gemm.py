@@ -62,6 +62,7 @@ def test_gemm_equals_oracle(S, rows, n_out, k):
     (2200, 2047, 512, False), (2113, 1985, 2048, True),                     # 64 x 32, halves
     (2689, 2999, 512, False), (2600, 2500, 2048, True),                     # 128 x 32, a tile past the padding
     (1024, 700, 256, False), (2560, 2700, 256, False), (3072, 2690, 768, False),  # an XCD's share of the tokens
+    (2600, 2500, 512, False), (2560, 2500, 256, False), (3072, 2600, 256, False),
     (100, 1100, 2048, True), (2177, 2200, 2048, True), (2689, 3333, 2048, True)])  # row tiles past whole eights
 def test_gemm_wavefront_tiles(S, rows, n_out, k, x8):
     """Each wavefront tile the product is dispatched to, at ragged sizes, over both weight orders."""
