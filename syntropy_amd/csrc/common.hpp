@@ -398,8 +398,8 @@ SYN_DEV uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(lds_ptr)
 // here; the second is also the wait state between a scalar write of m0 and the LDS DMA.
 // BARE: that wait state alone, for kernels whose assembly is checked to hold no such pair
 // (tests/test_lds_copy_wait_states.py).  The moves cost the kernels that wait on one chain of copies
-// and products 2 % (F16 4096 x 14336 at 9 rows 45.3 against 46.1 us, Q4_K 2048 x 8192 at 64 rows 37.1
-// against 38.0); five s_nop cost the int8 GEMMs 5 to 8 %.
+// and products 2 to 5 % (F16 4096 x 14336 at 9 rows 45.3 against 46.1 us, Q4_K 2048 x 8192 at 64 rows 37.1
+// against 38.0, Q4_K 2760 x 7936 at 2 rows 23.9 against 25.2); five s_nop cost the int8 GEMMs 5 to 8 %.
 template <bool BARE = false>
 SYN_DEV void lds_dma16(uint32_t voff, const void* sbase, uint32_t lds) {
     if constexpr (BARE) {
@@ -443,11 +443,18 @@ SYN_DEV void lds_dma4(uint32_t voff, const void* sbase, uint32_t lds) {
 }
 
 // As lds_dma16, from each lane's own address.
+template <bool BARE = false>
 SYN_DEV void lds_dma16_at(const void* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, m0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                 :
-                 : "v"(src), "{m0}"(lds)
-                 : "memory");
+    if constexpr (BARE)
+        asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                     :
+                     : "v"(src), "{m0}"(lds)
+                     : "memory");
+    else
+        asm volatile("s_mov_b32 m0, m0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                     :
+                     : "v"(src), "{m0}"(lds)
+                     : "memory");
 }
 
 }  // namespace syn

@@ -870,7 +870,7 @@ SYN_DEV void issue_slot(const Slot& sl, int b, uint8_t* stage) {
     if (sl.live && sl.on) {
         const uint8_t* src = sl.x8 ? sl.src + x8_chunk_offset(sl.xg0 + (uint32_t)b, sl.xq, sl.xnb)
                                    : sl.src + (uint64_t)sl.step * (uint32_t)b;
-        lds_dma16_at(src, lds_addr(stage + sl.lds));
+        lds_dma16_at<true>(src, lds_addr(stage + sl.lds));
     }
 }
 
