@@ -446,7 +446,8 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
                                 g.xd + x * (uint64_t)nb);
             }
         }
-        if constexpr (MODE != G32_DENSE) lds_barrier();  // the last stages are read out
+        const bool vec = (g.n_out & 3) == 0 && ((uintptr_t)g.y & 15) == 0;  // uniform
+        if (MODE != G32_DENSE || !vec) lds_barrier();  // the last stages are read out
         v16f_q up[TT];
         if constexpr (MODE == G32_GATEUP) {  // [wavefront][tile][i][lane]
             float* ux = reinterpret_cast<float*>(lds) + (size_t)(wave % (RG * TG)) * TT * 1024;
@@ -464,6 +465,34 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
             lds_barrier();  // read before another tile's copies
         }
         if (!busy || (C::R == 2 && mat)) continue;
+        if constexpr (MODE == G32_DENSE) {
+            // Rows of y that do not start at 16 bytes: the tile goes through the wavefront's part of LDS, so
+            // that 32 lanes write a token's 32 outputs side by side and not four bytes of 32 tokens (4098 x 512
+            // Q8_0 SPLIT at 1411 rows 27.5 against 37.1 us, of 4100 outputs 25.8).
+            if (!vec) {
+                static_assert(C::NW * 32 * 33 * 4 <= C::LDS, "the tiles fit the ring");
+                int id = lane;
+                asm volatile("" : "+v"(id));  // what follows from it is not computed before the loop, which has no registers left
+                const int col = id & 31, half = id >> 5, n = row0 + 32 * rg + col;
+                float* tx = reinterpret_cast<float*>(lds) + wave * 32 * 33;  // [token][row]
+#pragma unroll
+                for (int t = 0; t < TT; ++t) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) tx[33 * col + 4 * half + 8 * (i >> 2) + (i & 3)] = acc[t][i];
+                    __builtin_amdgcn_wave_barrier();
+                    const int first = 32 * (TT * tg + t);
+                    const int tokens = valid - first < 32 ? valid - first : 32;
+                    float* yr = g.y + (uint64_t)(t0 + first + half) * (uint64_t)g.n_out + (uint64_t)n;
+#pragma unroll 4
+                    for (int lt = half; lt < 32; lt += 2) {
+                        if (lt < tokens && n < g.n_out) *yr = tx[33 * lt + col];
+                        yr += 2 * (uint64_t)g.n_out;
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                }
+                continue;
+            }
+        }
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
             const int tt = 32 * (TT * tg + t) + c;
@@ -477,11 +506,10 @@ __global__ __launch_bounds__(64 * RG * TG * (MODE == G32_GATEUP ? 2 : 1), 2) voi
                                   : MODE == G32_GATEUP ? (uint64_t)(e0 + (uint32_t)tk)
                                                        : (uint64_t)g.slots[e0 + (uint32_t)tk];
             float* yr = g.y + yrow * (uint64_t)g.n_out;
-            const bool vec = (g.n_out & 3) == 0 && ((uintptr_t)g.y & 15) == 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int n = n0 + 8 * q;
-                if (vec) {
+                if (MODE == G32_DENSE || vec) {
                     if (n < g.n_out) *reinterpret_cast<float4*>(yr + n) = make_float4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
                 } else {
 #pragma unroll

@@ -168,3 +168,45 @@ def test_experts(S, E, top_k, hidden, inter, rows, popular):
     ex = M.Experts(M.WeightType.Q8_0, dev(gate), dev(up), dev(down))
     got = M.moe_grouped(M.MoeShape(E, top_k, hidden, inter), ex, dev(x), dev(ids))
     assert_same(host(got), want, "experts")
+
+
+@pytest.mark.parametrize("ty", [o.Q8_0, o.Q4_0])
+@pytest.mark.parametrize("rows,n_out,k,at", [(20, 100, 96, 1), (70, 68, 160, 2), (1025, 4100, 64, 3), (33, 31, 96, 0)])
+def test_outputs_at_any_address(S, ty, rows, n_out, k, at):
+    """Outputs that no row starts at 16 bytes of (the tile goes through LDS), one and two token tiles a
+    wavefront: the values, and nothing written beside them."""
+    rs = np.random.default_rng(rows + n_out + at)
+    w, x = blocks(rs, ty, n_out, k), rs.standard_normal((rows, k)).astype(np.float32)
+    want = o.gemv(ty, w, n_out, k, x, rows, threads=16)
+    W = S.Weights(S.WeightType(ty), dev(w), n_out, k)
+    for name, w_ in (("gguf", W), ("split", S.repack(W))):
+        buf = torch.full((rows * n_out + 64,), 7.5, device="cuda")
+        announce(f"q32 ty={ty} {name} {rows} {n_out}x{k} y at {at}")
+        S.gemv(w_, dev(x), rows, y=buf[at:at + rows * n_out])
+        got = host(buf)
+        assert_same(got[at:at + rows * n_out], want, f"{name} y at {at}")
+        assert (got[:at] == 7.5).all() and (got[at + rows * n_out:] == 7.5).all()
+
+
+@pytest.mark.parametrize("ty", [o.Q8_0, o.Q4_0])
+def test_ragged_outputs_take_no_longer(S, ty):
+    """1411 rows of 4098 outputs against 4100, as many tiles (measured: up to 1.1 times; four bytes of 32
+    rows at a time took 1.4 times)."""
+    k, rows = 512, 1411
+    rs = np.random.default_rng(31)
+    x = dev(rs.standard_normal((rows, k)).astype(np.float32))
+    Ws = [S.repack(S.Weights(S.WeightType(ty), dev(blocks(rs, ty, n, k)), n, k)) for n in (4100, 4098)]
+    ys = [torch.empty(rows, W.n_out, device="cuda") for W in Ws]
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    best = [float("inf")] * 2
+    announce(f"q32 ty={ty} ragged outputs")
+    for _ in range(8):
+        for i, W in enumerate(Ws):
+            ev[0].record()
+            for _ in range(10):
+                S.gemv(W, x, rows, y=ys[i])
+            ev[1].record()
+            torch.cuda.synchronize()
+            best[i] = min(best[i], 100 * ev[0].elapsed_time(ev[1]))
+    print(f"4100: {best[0]:.1f} us, 4098: {best[1]:.1f} us")
+    assert best[1] < 1.25 * best[0]
