@@ -273,7 +273,9 @@ constexpr int GF_WIDE_WGS = 129;
 // ends.  Up to four activation rows, rows of medium length too are better off with two workgroups of two
 // stages than with one of four.  Four stages of eight wavefronts | two of eight | two of four: one row of
 // 50000 x 768 21 | 16 | 15 us, 50000 x 2048 35 | 35 | 38, 32064 x 4096 46 | 43 | 52, 14336 x 14336 86 | 90 | 83;
-// 16 rows of 50000 x 768 38 | 35 | 30, 50000 x 4096 137 | 135 | 126.
+// 16 rows of 50000 x 768 38 | 35 | 30, 50000 x 4096 137 | 135 | 126.  (Rows of 32 to 128 values stay up to 15 %
+// slower at one row, and up to 10 % at 17 to 20, than one 16-byte load a lane and F32 FMAs: 100000 x 64 at one row
+// 8.7 against 7.9 us, at five 10.9 against 14.0.)
 constexpr int GF_SHORT = 1024, GF_MID = 4096;
 
 // Beyond 16 activation rows, groups of 16 (32 in one workgroup leave one wavefront a SIMD: 32064 x
@@ -288,7 +290,7 @@ static void launch_float_rows(const uint8_t* W, int n_out, int k, const float* x
             launch_float<BF16, VEC, 1, 2, 4, 256, 2>(W, n_out, k, x, rows, y, stream, active);
         else if (rows <= 8)
             launch_float<BF16, VEC, 2, 2, 4, 256, 2>(W, n_out, k, x, rows, y, stream, active);
-        else if (rows <= 12)
+        else if (rows <= 12 || (rows + 11) / 12 * 3 < (rows + 15) / 16 * 4)  // 17 to 24 rows: two groups of 12
             launch_float<BF16, VEC, 3, 2, 4, 256, 2>(W, n_out, k, x, rows, y, stream, active);
         else
             launch_float<BF16, VEC, 4, 2, 4, 256, 2>(W, n_out, k, x, rows, y, stream, active);

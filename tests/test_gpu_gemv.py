@@ -410,7 +410,7 @@ def test_float_gemv_tiles(S, ty, rows, n_out, k, scale):
 
 @pytest.mark.parametrize("ty", [o.F16, o.BF16])
 @pytest.mark.parametrize("rows,n_out,k,w_at,x_at", [
-    (1, 8200, 1024, 0, 0), (7, 8193, 8, 0, 0), (11, 8207, 1016, 0, 0), (20, 4100, 264, 0, 0), (4, 8300, 1032, 0, 0),
+    (1, 8200, 1024, 0, 0), (7, 8193, 8, 0, 0), (11, 8207, 1016, 0, 0), (20, 4100, 264, 0, 0), (4, 8300, 1032, 0, 0), (24, 4100, 72, 0, 0), (36, 3000, 520, 0, 0),
     (2, 8200, 4104, 0, 0), (1, 33, 1, 2, 4), (2, 70, 481, 0, 0), (4, 17, 1441, 6, 12), (7, 40, 960, 14, 0), (16, 21, 512, 0, 8),
     (20, 35, 1023, 2, 4), (3, 8300, 225, 10, 4), (6, 8257, 449, 0, 0), (12, 8193, 672, 2, 12), (17, 4200, 37, 4, 4)])
 def test_float_gemv_any_address(S, ty, rows, n_out, k, w_at, x_at):
