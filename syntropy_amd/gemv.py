@@ -76,14 +76,24 @@ class Weights:
         return self.k_in // self.ty.block_elems() * self.ty.block_bytes()
 
 
-@functools.lru_cache(maxsize=1024)
-def _need(name: str, *shape: int) -> int:
-    """What a workspace query of the C ABI answers: a function of its whole numbers alone, so a call
-    that repeats a shape does not ask again (a one-row Gemv's host time 10 -> 7 us with the stream's
-    handle taken directly)."""
+def _ask(name: str, *shape: int) -> int:
     out = C.c_uint64()
     call(name, *shape, C.byref(out))
     return out.value
+
+
+_asked = functools.lru_cache(maxsize=1024)(_ask)
+
+
+def _need(name: str, *shape: int) -> int:
+    """What a workspace query of the C ABI answers: a function of its whole numbers alone, so a call
+    that repeats a shape does not ask again (a one-row Gemv's host time 10 -> 7 us with the stream's
+    handle taken directly).  Only plain whole numbers are kept: a float that equals one is refused as it
+    is when asked, and a tensor of one value, which hashes by identity, may change."""
+    for v in shape:
+        if v.__class__ is not int:
+            return _ask(name, *shape)
+    return _asked(name, *shape)
 
 
 def workspace_bytes(ty: WeightType, rows: int, k: int) -> int:
