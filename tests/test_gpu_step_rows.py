@@ -8,6 +8,8 @@ import pytest
 from gpu_util import announce, assert_same, dev
 from oracle import oracle as o
 from refgen import GemvRng, MoeRng, gemv_activations, gemv_weights, moe_matrix
+from test_gpu_gemm import random_q4k
+from test_gpu_gemm_q32 import blocks
 from test_gpu_provider import cx, gemv_key, shape  # noqa: F401  (the provider context fixture)
 
 pytestmark = pytest.mark.gpu
@@ -54,7 +56,7 @@ def dense_launch(cx, key, rows, n_out, k, w, x, step, y_cols=None):
 
 @pytest.mark.parametrize("ty,bucket,n_out,k,active", [
     (o.Q4_K, 8, 512, 2048, 5),    # the grouped-row kernel
-    (o.Q8_0, 12, 300, 1024, 9),   # two 8-row launches, the second with one active row
+    (o.Q8_0, 12, 300, 1024, 9),   # twelve rows on the int8 matrix cores, nine of them active
     (o.Q4_K, 1, 1024, 4096, 0),   # single-row decode, nothing active
     (o.Q4_K, 1, 1024, 4096, 1),
     (o.Q4_K, 64, 256, 4096, 40),  # the matrix-core GEMM
@@ -138,6 +140,102 @@ def test_gate_up_act_rows_active(cx):
     announce("rows_active gate_up_act")
     got = dense_launch(cx, key, bucket, n, k, w, x, step)
     check_rows(got, o.gate_up_act(o.Q4_K, w, n, k, x[:active], active, threads=8), active, "gate_up_act")
+
+
+def repacked(cx, key, w):
+    """(key, bytes) of the weights in the provider's own layout."""
+    import ctypes as C
+    import json
+    kb = json.dumps(key).encode()
+    kbuf = (C.c_uint8 * len(kb)).from_buffer_copy(kb)
+    present, lay = C.c_uint32(), C.c_uint32()
+    wl = np.zeros_like(w)
+    pr = cx.pr
+    pr.vt.repack(pr.vt.slf, kbuf, len(kb), w.ctypes.data_as(C.POINTER(C.c_uint8)), w.size,
+                 wl.ctypes.data_as(C.POINTER(C.c_uint8)), wl.size, C.byref(present), C.byref(lay))
+    return dict(key, layout=lay.value), wl
+
+
+@pytest.mark.parametrize("ty,packed,bucket,n_out,k,actives", [
+    (o.Q4_K, False, 1000, 3201, 256, (1, 640, 700)),     # 64 tokens x 32 rows a wavefront
+    (o.Q4_K, False, 2560, 2500, 256, (0, 1100, 1280)),   # an XCD's share of the tokens
+    (o.Q4_K, False, 3072, 2600, 256, (0, 1100, 2304)),   # the same at 128 tokens a workgroup
+    (o.Q4_K, False, 2600, 2500, 256, (129, 2599)),       # 128 tokens, a tile past the padding
+    (o.Q4_K, True, 2177, 2200, 2048, (0, 700)),          # row tiles past whole eights
+    (o.Q8_0, False, 200, 70, 160, (0, 3, 65)), (o.Q4_0, False, 70, 100, 96, (33,)),  # int8 matrix cores, GGUF order
+    (o.Q8_0, True, 1025, 4099, 160, (0, 40, 1024)), (o.Q4_0, True, 1025, 4100, 160, (63,))])  # SPLIT, two token tiles
+def test_many_row_gemv_rows_active(cx, ty, packed, bucket, n_out, k, actives):
+    """The many-row products with fewer rows active than the bucket, on and off a tile's edge."""
+    rs = np.random.default_rng(bucket + n_out + ty)
+    w = random_q4k(rs, n_out, k) if ty == o.Q4_K else blocks(rs, ty, n_out, k)
+    x = rs.standard_normal((bucket, k)).astype(np.float32)
+    want = o.gemv(ty, w, n_out, k, x[:max(actives)], max(actives), threads=16)
+    key, wl = repacked(cx, gemv_key(ty), w) if packed else (gemv_key(ty), w)
+    for active in actives:
+        _, step = step_desc(cx, active)
+        announce(f"rows_active gemv ty={ty} packed={packed} bucket={bucket} active={active}")
+        check_rows(dense_launch(cx, key, bucket, n_out, k, wl, x, step), want, active, f"gemv ty={ty} {active}")
+
+
+@pytest.mark.parametrize("ty", ["F16", "BF16"])
+@pytest.mark.parametrize("bucket,n_out,k,actives", [(20, 4100, 264, (5, 12, 13)), (40, 9000, 1056, (0, 16, 33)),
+                                                    (9, 40, 77, (4, 8))])
+def test_float_gemv_rows_active(cx, ty, bucket, n_out, k, actives):
+    """Groups of 12 and of 16 rows, rows of any length: whole groups and parts of one past rows_active."""
+    rs = np.random.default_rng(bucket + n_out)
+    f = rs.standard_normal(n_out * k).astype(np.float32)
+    w = (f.astype(np.float16) if ty == "F16" else (f.view(np.uint32) >> 16).astype(np.uint16)).view(np.uint8)
+    x = rs.standard_normal((bucket, k)).astype(np.float32)
+    want = o.gemv(getattr(o, ty), w, n_out, k, x[:max(actives)], max(actives), threads=16)
+    key = {"op": "Gemv", "schemes": [{"Plain": ty}, {"Plain": "F32"}, {"Plain": "F32"}], "layout": 0, "variant": 0}
+    for active in actives:
+        _, step = step_desc(cx, active)
+        announce(f"rows_active gemv {ty} bucket={bucket} active={active}")
+        check_rows(dense_launch(cx, key, bucket, n_out, k, w, x, step), want, active, f"gemv {ty} {active}")
+
+
+@pytest.mark.parametrize("packed,bucket,n,k,actives", [
+    (False, 1000, 1805, 256, (0, 640, 700)), (False, 2600, 1250, 256, (1, 1100)),  # 64 and 128 tokens a workgroup
+    (False, 3072, 1300, 256, (1100,)), (True, 993, 1601, 2048, (65,))])            # an XCD's share; row tiles past whole eights
+def test_gate_up_in_one_product_rows_active(cx, packed, bucket, n, k, actives):
+    rs = np.random.default_rng(bucket + n)
+    w = random_q4k(rs, 2 * n, k)
+    x = (0.1 * rs.standard_normal((bucket, k))).astype(np.float32)
+    want = o.gate_up_act(o.Q4_K, w, n, k, x[:max(actives)], max(actives), threads=16)
+    key = dict(gemv_key(o.Q4_K), op={"GateUpAct": {"act": "Silu"}})
+    key, wl = repacked(cx, key, w) if packed else (key, w)
+    for active in actives:
+        _, step = step_desc(cx, active)
+        announce(f"rows_active gate_up packed={packed} bucket={bucket} active={active}")
+        check_rows(dense_launch(cx, key, bucket, n, k, wl, x, step), want, active, f"gate_up {active}")
+
+
+@pytest.mark.parametrize("E,top_k,hidden,inter,bucket,actives", [(6, 2, 256, 512, 300, (200, 0)), (16, 4, 96, 160, 20, (9,))])
+def test_q8_0_experts_rows_active(cx, E, top_k, hidden, inter, bucket, actives):
+    """Q8_0 experts, whose rows are quantized before the entries are known: NaN rows and ids out of range
+    past rows_active."""
+    P, pr = cx.P, cx.pr
+    rs = np.random.default_rng(E + bucket)
+    gate, up, down = (blocks(rs, o.Q8_0, E * n, k) for n, k in ((inter, hidden), (inter, hidden), (hidden, inter)))
+    x0 = rs.standard_normal((bucket, hidden)).astype(np.float32)
+    ids0 = np.stack([rs.permutation(E)[:top_k] for _ in range(bucket)]).astype(np.int32)
+    key = {"op": "MoeGrouped", "schemes": [{"Ggml": "Q8_0"}, {"Plain": "F32"}, {"Plain": "F32"}], "layout": 0,
+           "variant": 0}
+    op = pr.prepare(cx.ctx, key, shape(bucket, E, top_k, hidden, inter))
+    mats = [dev(m) for m in (gate, up, down)]
+    for active in actives:
+        x, ids = x0.copy(), ids0.copy()
+        x[active:], ids[active:] = np.nan, 999
+        _, step = step_desc(cx, active)
+        announce(f"rows_active q8_0 experts E={E} bucket={bucket} active={active}")
+        xb, ids_b, per_b = cx.put(x), cx.put(ids), cx.empty(4 * bucket * top_k * hidden)
+        pr.launch(cx.ctx, cx.s, op, P.op_args(
+            [P.packed(xb, P.DT_F32, [bucket, hidden]), P.packed(ids_b, P.DT_I32, [bucket, top_k])],
+            [P.packed(per_b, P.DT_F32, [bucket, top_k, hidden])], [P.view(t.data_ptr(), t.numel()) for t in mats],
+            cx.workspace(op), step=step))
+        want = o.moe_grouped(o.Q8_0, o.Q8_0, E, top_k, hidden, inter, gate, up, down, x[:active], ids[:active],
+                             threads=8).reshape(active, top_k * hidden) if active else None
+        check_rows(cx.get(per_b, np.float32, (bucket, top_k * hidden)), want, active, f"q8_0 experts {active}")
 
 
 @pytest.mark.parametrize("E,top_k,hidden,inter,bucket,active", [
