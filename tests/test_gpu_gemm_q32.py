@@ -210,3 +210,60 @@ def test_ragged_outputs_take_no_longer(S, ty):
             best[i] = min(best[i], 100 * ev[0].elapsed_time(ev[1]))
     print(f"4100: {best[0]:.1f} us, 4098: {best[1]:.1f} us")
     assert best[1] < 1.25 * best[0]
+
+
+@pytest.mark.parametrize("k,rows", [(4128, 9), (4096, 40), (4128, 70), (4096, 130)])
+def test_split_matrix_past_32_bit_offsets(S, k, rows):
+    """A Q8_0 SPLIT matrix of more than 4 GiB, which the register-staged kernel takes (16 and 32 tokens a
+    tile, rows of whole and of odd stages): slices at both ends and around the 4 GiB mark."""
+    n_out, nb = 1_050_003, k // 32
+    g = torch.Generator("cuda").manual_seed(k + rows)
+    buf = torch.empty(n_out * nb * 34, dtype=torch.uint8, device="cuda")
+    codes, scales = buf[:n_out * k], buf[n_out * k:].view(torch.int16)
+    for a in range(0, codes.numel(), 1 << 30):
+        codes[a:a + (1 << 30)].random_(0, 256, generator=g)
+    scales.random_(3 << 10, 13 << 10, generator=g)
+    x = torch.randn(rows, k, generator=g, device="cuda")
+    announce(f"q8_0 split {n_out}x{k} rows {rows}")
+    y = S.gemv(S.Weights(S.WeightType.Q8_0, buf, n_out, k, S.LAYOUT_SPLIT), x, rows)
+    for a in (0, (1 << 32) // k - 16, n_out - 33):
+        w = np.empty((33, nb, 34), np.uint8)
+        w[:, :, 2:] = host(codes[a * k:(a + 33) * k]).reshape(33, nb, 32)
+        w[:, :, :2] = host(scales[a * nb:(a + 33) * nb]).view(np.uint8).reshape(33, nb, 2)
+        want = o.gemv(o.Q8_0, w.reshape(-1), 33, k, host(x), rows, threads=16)
+        assert_same(host(y[:, a:a + 33].contiguous()), want, f"outputs from {a}")
+
+
+@pytest.mark.parametrize("hidden,inter", [(61_696, 65_536), (61_728, 65_504)])  # rows of whole 16-byte pieces, or not
+def test_expert_past_32_bit_offsets(S, hidden, inter):
+    """One Q8_0 expert whose matrices hold about 4 GiB each, past gemm_q32.hip's 32-bit offsets, against the
+    dense ops over row slices."""
+    import syntropy_amd.moe as M
+    rows, part = 3, 8192
+    g = torch.Generator("cuda").manual_seed(41)
+
+    def matrix(n, k):
+        m = torch.empty(n * (k // 32) * 17, dtype=torch.int16, device="cuda")
+        for a in range(0, m.numel(), 1 << 30):
+            m[a:a + (1 << 30)].random_(generator=g)
+        m.view(-1, 17)[:, 0].random_(1 << 10, 5 << 10, generator=g)
+        return m.view(torch.uint8)
+
+    gate, up, down = matrix(inter, hidden), matrix(inter, hidden), matrix(hidden, inter)
+    assert gate.numel() >= (1 << 32) - 65536
+    x = torch.randn(rows, hidden, generator=g, device="cuda")
+    ids = torch.zeros(rows, 1, dtype=torch.int32, device="cuda")
+    announce(f"q8_0 expert {inter}x{hidden}")
+    got = M.moe_grouped(M.MoeShape(1, 1, hidden, inter), M.Experts(M.WeightType.Q8_0, gate, up, down), x, ids)
+    assert torch.isfinite(got).all()
+    h = torch.empty(rows, inter, device="cuda")
+    rb = hidden // 32 * 34
+    for a in range(0, inter, part):
+        n = min(part, inter - a)
+        w = torch.cat([gate[a * rb:(a + n) * rb], up[a * rb:(a + n) * rb]])
+        h[:, a:a + n] = S.gate_up_act(S.Weights(S.WeightType.Q8_0, w, 2 * n, hidden), x, rows)
+    rb = inter // 32 * 34
+    for a in range(0, hidden, part):
+        n = min(part, hidden - a)
+        want = S.gemv(S.Weights(S.WeightType.Q8_0, down[a * rb:(a + n) * rb].clone(), n, inter), h, rows)
+        assert_same(host(got.view(rows, hidden)[:, a:a + n].contiguous()), host(want), f"outputs from {a}")
