@@ -420,7 +420,7 @@ def bench_cfgs(torch, S, a):
         else:
             alg, kt = wb + T * (k + 8 * (k // 32)) + 4 * T * n, kern
         rows_res[str(T)] = {"kernel": "k_gemv_split<Q8_0,1,2> (row quantized in the workgroups)" if T == 1
-                            else "k_gemm_q8_staged",
+                            else "k_gemm_q32" if T > 32 else "k_gemm_q8_staged",
                             "step_us": round(step, 3), "weight_gbs": round(wb / (step * 1e-6) / 1e9, 1),
                             "kernel_us": round(kt, 3), "kernel_alg_gbs": round(alg / (kt * 1e-6) / 1e9, 1),
                             "kernel_frac": round(alg / (kt * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),

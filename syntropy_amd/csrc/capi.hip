@@ -603,9 +603,9 @@ SYN_EXPORT int syn_split_repack_host(uint32_t layout, int32_t wtype, const void*
 // Gemv over weights in a repacked layout.  Q4_K in X8: one row runs the grouped decode kernel,
 // 2 to 31 rows the decode expert kernel (int8 matrix cores), more rows the matrix-core GEMM (which
 // needs rows of whole 8-block runs: k_in a multiple of 2048).  Q8_0 / Q4_0 in SPLIT: Q8_0 activation
-// rows, the split decode kernel for up to 8 rows at a time, the int8 matrix-core GEMM where its
-// LDS-staged form takes the shape (rows of whole 4-block stages) and is the faster, and for other
-// Q8_0 shapes from 9 rows.
+// rows, the split decode kernel for up to 8 rows at a time, the int8 matrix-core GEMMs where they are
+// the faster (split_gemm): over rows of whole 4-block stages from 2 rows on, over others Q8_0 from 9
+// and Q4_0 from a count that follows the row length.
 constexpr uint32_t SPLIT_GEMM_MIN_ROWS = 9;
 constexpr uint32_t SPLIT_GEMM_MAX_ROWS = 65535u * 32u;  // the GEMM grid's token tiles
 

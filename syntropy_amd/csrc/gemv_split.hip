@@ -16,11 +16,12 @@
 // 128 blocks at a time: one fold instruction serves every row of the workgroup (a lane-0-only
 // fold per wavefront costs as many instructions as all the row's other arithmetic together).
 //
-// 2 or more rows (k_gemm_q8_splitk up to 16 rows of whole 16-block stages, k_gemm_q8_staged for
-// more rows or rows of whole 4-block stages, Q8_0 and Q4_0; else for Q8_0 from 9 rows
-// k_gemm_q8_split): v_mfma_i32_16x16x32_i8 takes one 32-value block of 16 weight rows against 16
-// tokens: the exact I32 sums of 256 outputs, which are scaled and folded (one term per block, in
-// block order).
+// 2 or more rows of whole 4-block stages, while the outputs are fewer than gemm_q32.hip's tiles take
+// (launch_gemm_q8_split): k_gemm_q8_splitk up to 32 rows of whole 16-block stages where it is estimated
+// the faster, else k_gemm_q8_staged.  k_gemm_q8_split: Q8_0 matrices or activations past the 32-bit
+// offsets of both files' other kernels.  v_mfma_i32_16x16x32_i8 takes one 32-value block of 16 weight
+// rows against 16 tokens: the exact I32 sums of 256 outputs, which are scaled and folded (one term per
+// block, in block order).
 #include <type_traits>
 
 #include "common.hpp"
@@ -1043,8 +1044,8 @@ static void launch_staged_fmt(const uint8_t* W, int n_out, int k, const int8_t* 
     }
 }
 
-// Q8_0 rows of any shape (the staged GEMM where it fits, else the register-staged one); Q4_0 rows
-// where the staged GEMM fits (gemm_q8_staged_fits).
+// Q8_0 rows of any shape; Q4_0 rows where gemm_q32.hip or the staged GEMM fits (gemm_q32_fits,
+// gemm_q8_staged_fits).
 void launch_gemm_q8_split(int ty, const uint8_t* W, int n_out, int k, const uint8_t* ws, int T, float* y,
                           hipStream_t stream, const uint32_t* active) {
     const ActLayout L = act_layout(ACT_Q8_0, (uint64_t)T, (uint64_t)k);
