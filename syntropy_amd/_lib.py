@@ -100,7 +100,7 @@ def bind(name: str, argtypes, restype=C.c_int):
 
 
 def call(name: str, *args) -> None:
-    rc = getattr(lib(), name)(*args)
+    rc = getattr(_lib if _lib is not None else lib(), name)(*args)
     if rc != 0:
         raise SynError(rc, lib().syn_last_error().decode())
 

@@ -82,7 +82,15 @@ def _ask(name: str, *shape: int) -> int:
     return out.value
 
 
-_asked = functools.lru_cache(maxsize=1024)(_ask)
+class _NotKept(Exception):
+    pass
+
+
+@functools.lru_cache(maxsize=1024, typed=True)
+def _kept(name: str, *shape: int) -> int:
+    if any(v.__class__ is not int for v in shape):
+        raise _NotKept  # which the cache does not keep
+    return _ask(name, *shape)
 
 
 def _need(name: str, *shape: int) -> int:
@@ -90,10 +98,10 @@ def _need(name: str, *shape: int) -> int:
     that repeats a shape does not ask again (a one-row Gemv's host time 10 -> 7 us with the stream's
     handle taken directly).  Only plain whole numbers are kept: a float that equals one is refused as it
     is when asked, and a tensor of one value, which hashes by identity, may change."""
-    for v in shape:
-        if v.__class__ is not int:
-            return _ask(name, *shape)
-    return _asked(name, *shape)
+    try:
+        return _kept(name, *shape)
+    except _NotKept:
+        return _ask(name, *shape)
 
 
 def workspace_bytes(ty: WeightType, rows: int, k: int) -> int:
@@ -167,16 +175,17 @@ def gemv(w: Weights, x: torch.Tensor, rows: int, y: torch.Tensor | None = None,
         y = torch.empty(rows, w.n_out, dtype=torch.float32, device=x.device)
     elif y.numel() < rows * w.n_out:
         raise GemvError("Len", f"`y` holds {y.numel()} values, the op needs {rows * w.n_out}")
+    ty, wb = int(w.ty), w.bytes
     if w.layout != LAYOUT_SOURCE:
         if ws is None:
-            need = _need("syn_gemv_layout_workspace_bytes", w.layout, int(w.ty), rows, w.k_in)
+            need = _need("syn_gemv_layout_workspace_bytes", w.layout, ty, rows, w.k_in)
             ws = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device)
-        call("syn_gemv_layout", w.layout, int(w.ty), w.bytes.data_ptr(), w.bytes.numel(), w.n_out, w.k_in,
+        call("syn_gemv_layout", w.layout, ty, wb.data_ptr(), wb.numel(), w.n_out, w.k_in,
              x.data_ptr(), rows, y.data_ptr(), ws.data_ptr(), ws.numel(), _stream(stream))
         return y
     if ws is None:
         ws = new_workspace(w.ty, rows, w.k_in, x.device)
-    call("syn_gemv", int(w.ty), w.bytes.data_ptr(), w.bytes.numel(), w.n_out, w.k_in,
+    call("syn_gemv", ty, wb.data_ptr(), wb.numel(), w.n_out, w.k_in,
          x.data_ptr(), rows, y.data_ptr(), ws.data_ptr(), ws.numel(), _stream(stream))
     return y
 
