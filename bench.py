@@ -427,7 +427,8 @@ def bench_cfgs(torch, S, a):
                             "tflops": round(2.0 * T * n * k / (step * 1e-6) / 1e12, 2)}
         if T > 1:
             # the F32 term of every (output, block): convert, two multiplies, add (gemv.rs:539-547),
-            # one VALU lane-operation each, against the VALU issue peak
+            # one VALU lane-operation each as the reference writes them (k_gemm_q32 has two of them
+            # done by the matrix cores), against the VALU issue peak
             ops = 4.0 * T * n * (k // 32)
             rows_res[str(T)]["valu_roofline"] = {
                 "bound": "valu", "ops_per_launch": int(ops), "unit": "T lane-ops/s",
